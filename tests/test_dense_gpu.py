@@ -1,0 +1,84 @@
+"""The dense bf16 route (dense_fast.hip) over its tile heights, ring
+remainders and tails: against the oracle at the projection bar (2e-3, the
+output's one bf16 rounding being 1.66e-3), and bit for bit against the general
+kernel, which multiplies in the same k16 order and rounds once too."""
+import numpy as np
+import pytest
+
+import ming_dit_amd as m
+from helpers import bf16, empty_bf16, from_dev, make_lora, make_weight, randn, sync, to_dev
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-3
+
+
+def _run(ctx, route, fn, M, N, ldy=None):
+    ctx.set_route(route)
+    y = empty_bf16(M, ldy or N)
+    y.zero_()
+    sync()
+    fn(y)
+    sync()
+    ctx.set_route("auto")
+    return from_dev(y)
+
+
+# N % 64 != 0 (or a live adapter) keeps a small grid off the split-K GEMM.
+# 64-row tiles while they fit one round of 256 blocks, taller ones past it.
+@pytest.mark.parametrize("M,N,K,ranks", [
+    (9, 264, 64, ()),                  # one stage, one ragged row tile
+    (65, 264, 128, (8,)),              # two stages; an odd tail of one chunk
+    (200, 1000, 192, (32, 32)),        # a tail of two chunks, ragged columns
+    (130, 520, 320, (4, 40, 64)),      # five stages; four chunks
+    (2085, 2056, 384, (16, 64)),       # 128-row tiles; three chunks
+    (4300, 2048, 448, (64, 64, 48)),   # 192-row tiles; six chunks, seven stages
+    (6210, 2048, 256, (33,)),          # 256-row tiles; two chunks
+])
+def test_dense_route(ctx, orc, M, N, K, ranks):
+    print(f"case dense M={M} N={N} K={K} ranks={ranks}", flush=True)
+    x = bf16(randn(9000 + M, (M, K)))
+    pack, w = make_weight(9100 + N, N, K, 16, std=1.0 / np.sqrt(K))
+    qw = m.QWeight.dense(ctx, pack["w"])
+    scales, loras = [0.0] * 8, []
+    for i, r in enumerate(ranks):
+        A, B = make_lora(9200 + 2 * i, N, K, r)
+        qw.bind_lora(i, A, B)
+        scales[i] = 0.7 - 0.4 * i
+        loras.append((A, B, scales[i]))
+    xd = to_dev(x)
+    got, want = (_run(ctx, r, lambda y: ctx.lin(qw, xd, y, M, scales), M, N)
+                 for r in ("auto", "general"))
+    ref = orc.proj(x, w, loras)
+    assert orc.rel_l2(orc.bf16_to_f32(got), ref) <= TOL
+    if ranks:
+        # the two routes slice the x.A differently: T may differ by a bf16 ulp
+        assert orc.rel_l2(orc.bf16_to_f32(got), orc.bf16_to_f32(want)) <= 1e-3
+        got, want = (_run(ctx, r, lambda y: ctx.lin(qw, xd, y, M), M, N)
+                     for r in ("auto", "general"))
+    assert np.array_equal(got, want)
+    # the fused bias and SwiGLU, and an output stride that leaves 8-byte rows
+    bias, gate = to_dev(bf16(randn(9300, (N,)))), to_dev(bf16(randn(9301, (M, N))))
+    for ldy, fn in ((N, lambda y: ctx.lin_bias(qw, xd, y, M, bias)),
+                    (N, lambda y: ctx.lin_swiglu(qw, xd, gate, y, M)),
+                    (N + 4, lambda y: ctx.lin(qw, xd, y, M, ldy=N + 4))):
+        a, b = (_run(ctx, r, fn, M, N, ldy) for r in ("auto", "general"))
+        assert np.array_equal(a, b)
+    qw.close()
+
+
+@pytest.mark.parametrize("M", [40, 300])
+def test_dense_gated_few_tiles(ctx, M):
+    """A gated dense projection of few tiles gives ming_lin's bits, then
+    ming_swiglu's, whichever kernel ming_lin takes."""
+    N, K = 512, 2048
+    pack, _ = make_weight(9400, N, K, 16, std=1.0 / np.sqrt(K))
+    qw = m.QWeight.dense(ctx, pack["w"])
+    xd, g = to_dev(bf16(randn(9401, (M, K)))), to_dev(bf16(randn(9402, (M, N))))
+    u, want, got = empty_bf16(M, N), empty_bf16(M, N), empty_bf16(M, N)
+    sync()
+    ctx.lin(qw, xd, u, M)
+    ctx.swiglu(g, u, want, M, N)
+    ctx.lin_swiglu(qw, xd, g, got, M)
+    sync()
+    assert np.array_equal(from_dev(got), from_dev(want))
+    qw.close()

@@ -73,7 +73,7 @@ struct QprojArgs {
   const uint32_t* sb_u;
   QprojSeg seg_u;
   // optional bias [N] bf16, added to the f32 result before the output's one
-  // bf16 rounding (the general kernel: a dense weight's ming_lin_bias)
+  // bf16 rounding (dense weights: ming_lin_bias)
   const uint16_t* bias;
 };
 
@@ -294,6 +294,17 @@ hipError_t launch_lora_xa_fast(const LoraXaArgs& a, float* part, int kslices,
 hipError_t launch_bf16_to_f16(const uint16_t* x, long long ldx, uint16_t* y,
                               long long ldy, int rows, int K, hipStream_t s,
                               int* range = nullptr);
+
+// ---- the dense bf16 route (dense_fast.hip) ------------------------------------
+// y = x . W^T (+ the LoRA tail), W = a.w16 [N][K] bf16, x bf16 at ldx, with
+// a.bias or a.g (fused SwiGLU) as QprojArgs says. N % 8 == 0, K % 64 == 0; x,
+// W, T and every B stack within 2 GiB of their base. rf: 64*rf rows a tile.
+hipError_t launch_dense_fast(const QprojArgs& a, int rf, hipStream_t s);
+// The tile height (rf) for a shape, and whether a dense projection of few
+// tiles is better split along K (launch_lora_xa_fast, identity groups).
+int dense_fast_rf(int M, int N);
+bool dense_prefers_split(int M, int N, int K);
+hipError_t validate_dense_fast_kernels();
 
 hipError_t validate_qproj_kernels();
 hipError_t validate_qproj_fast_kernels();

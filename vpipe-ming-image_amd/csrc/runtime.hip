@@ -451,6 +451,7 @@ int ming_ctx_create(int device, void* hip_stream, ming_ctx** out) {
   if (e == hipSuccess) e = ming::validate_norm_kernels();
   if (e == hipSuccess) e = ming::validate_elementwise_kernels();
   if (e == hipSuccess) e = ming::validate_qproj_fast_kernels();
+  if (e == hipSuccess) e = ming::validate_dense_fast_kernels();
   if (e == hipSuccess) e = ming::validate_gemv_kernels();
   if (e == hipSuccess) e = ming::validate_attention_kernels();
   if (e != hipSuccess)
@@ -1008,16 +1009,17 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
   // 64-bit base plus 32-bit byte offsets: x (fp16 copy, row stride K), T and
   // every B stack must fit.
   bool fast[ming::kMaxXaSources] = {};
+  bool tail_fits[ming::kMaxXaSources] = {};   // T and the B stacks
   bool any_fast = false;
   for (int i = 0; i < n; ++i) {
     const ming_qweight* q = qs[i];
-    bool fits32 = (uint64_t)M * (uint64_t)K * 2 <= (1ull << 31) &&
-                  (uint64_t)M * (uint64_t)t_cols * 2 <= (1ull << 31);
+    tail_fits[i] = (uint64_t)M * (uint64_t)t_cols * 2 <= (1ull << 31);
     for (int si = 0; si < (int)q->segs.size() && t_cols > 0; ++si)
       if (qa[i].seg[si].chunks > 0 &&
           (uint64_t)q->segs[si].N * (uint64_t)q->b_ld[si] * 2 > (1ull << 31))
-        fits32 = false;
-    fast[i] = q->bits != 16 && q->fast && c->route == MING_ROUTE_AUTO && fits32;
+        tail_fits[i] = false;
+    fast[i] = q->bits != 16 && q->fast && c->route == MING_ROUTE_AUTO && tail_fits[i] &&
+              (uint64_t)M * (uint64_t)K * 2 <= (1ull << 31);
     any_fast = any_fast || fast[i];
   }
   // Per projection: the fast route's K split on few tiles (the context
@@ -1025,10 +1027,14 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
   // chip at >= 6 K steps a slice; a dense weight with no live adapter on few
   // 256 x 256 tiles (the caption embedder: 15; the final layer's 64
   // columns: 16) runs as the x.A path's split-K bf16 GEMM (identity column
-  // groups, coefficient 1); the general route writes a gated projection into
-  // a plane of its own first, since y may be the gate itself.
+  // groups, coefficient 1) where that is the faster one; it and the general
+  // route write a gated projection into a plane of its own first, since y may
+  // be the gate itself.
   int split_ks[ming::kMaxXaSources] = {};
   int dense_ks[ming::kMaxXaSources] = {};
+  // every other dense projection: the dense route's tile height, 0 where its
+  // 32-bit offsets or its 8-column stores do not fit (the general kernel)
+  int dense_rf[ming::kMaxXaSources] = {};
   size_t up_bytes = 0;
   for (int i = 0; i < n; ++i) {
     const ming_qweight* q = qs[i];
@@ -1042,16 +1048,18 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
         part_bytes = std::max(part_bytes, (size_t)ks * M * q->N * 4);
       }
     }
-    const bool dense_sk =
-        q->bits == 16 && c->route != MING_ROUTE_GENERAL && live_segs[i] == 0 && !o.gate &&
-        !o.yh && tiles < 64 && q->N % 64 == 0 && q->N <= 8 * ming::kMaxGroups &&
-        K % 64 == 0 && o.ldy <= (1 << 30) && (uint64_t)M * (uint64_t)ldx * 2 <= (1ull << 31) &&
-        (uint64_t)q->N * (uint64_t)K * 2 <= (1ull << 31);
-    if (dense_sk) {
+    const bool dense = q->bits == 16 && c->route != MING_ROUTE_GENERAL &&
+                       (uint64_t)M * (uint64_t)ldx * 2 <= (1ull << 31) &&
+                       (uint64_t)q->N * (uint64_t)K * 2 <= (1ull << 31);
+    if (dense && live_segs[i] == 0 && tiles < 64 && q->N % 64 == 0 &&
+        q->N <= 8 * ming::kMaxGroups && K % 64 == 0 && o.ldy <= (1 << 30) &&
+        ming::dense_prefers_split(M, q->N, K)) {
       dense_ks[i] = ming::dense_xa_slices(M, q->N, K);
       part_bytes = std::max(part_bytes, ming::lora_xa_part_bytes(M, q->N, dense_ks[i]));
+    } else if (dense && q->N % 8 == 0 && tail_fits[i]) {
+      dense_rf[i] = ming::dense_fast_rf(M, q->N);
     }
-    if (o.gate && !fast[i]) up_bytes = std::max(up_bytes, (size_t)M * q->N * 2);
+    if (o.gate && !fast[i] && !dense_rf[i]) up_bytes = std::max(up_bytes, (size_t)M * q->N * 2);
   }
   // A SwiGLU's gate and up projections (the second gated by the first's
   // output, as ming_ffn runs w1 and w3) on the fast route run as one launch:
@@ -1178,9 +1186,13 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
     a.g = nullptr; a.ldg = 0;
     a.yh = nullptr; a.ldyh = 0;
     a.range = range_word(c);
-    a.bias = o.bias;   // set for dense weights only: the general kernel adds it
-    if (o.gate && !fast[i]) {
+    a.bias = o.bias;   // set for dense weights only
+    const bool fused_gate = fast[i] || dense_rf[i] > 0;
+    if (o.gate && !fused_gate) {
       a.y = up; a.ldy = q->N;
+    }
+    if (dense_rf[i]) {
+      a.g = o.gate; a.ldg = o.ldg;
     }
     if (fast[i]) {
       a.x = xh; a.ldx = K; a.codes = q->codes_f; a.sb = q->sbf;
@@ -1200,7 +1212,7 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
     if (dense_ks[i] > 0) {
       ming::LoraXaArgs da{};
       da.x = x; da.ldx = ldx; da.A[0] = q->w16; da.K = K; da.M = M;
-      da.n_cols = q->N; da.t = o.y; da.ldt = (int)o.ldy; da.bias = o.bias;
+      da.n_cols = q->N; da.t = a.y; da.ldt = (int)a.ldy; da.bias = o.bias;
       for (int gi = 0; gi < q->N / 8; ++gi) {
         da.grp[gi] = (int16_t)gi;
         da.coef[gi] = 1.0f;
@@ -1213,13 +1225,14 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
       MING_HIP(profiled(c, bk, base_flops + tail_flops[i],
                         2.0 * M * K + wbytes + 2.0 * M * q->N,
                         [&] {
-                          return fast[i] ? ming::launch_qproj_fast(q->bits, a, c->stream)
-                                         : ming::launch_qproj(q->bits, a, c->stream,
-                                                              c->route == MING_ROUTE_WIDE);
+                          return fast[i]       ? ming::launch_qproj_fast(q->bits, a, c->stream)
+                                 : dense_rf[i] ? ming::launch_dense_fast(a, dense_rf[i], c->stream)
+                                               : ming::launch_qproj(q->bits, a, c->stream,
+                                                                    c->route == MING_ROUTE_WIDE);
                         }),
                "qproj launch");
     }
-    if (o.gate && !fast[i]) {
+    if (o.gate && !fused_gate) {
       // the general route writes the projection; SwiGLU follows
       MING_HIP(profiled(c, kBSwiglu, 0.0, 6.0 * M * q->N,
                         [&] { return ming::launch_swiglu(o.gate, o.ldg, up, q->N, o.y,
