@@ -61,6 +61,7 @@ struct QprojArgs {
   // summed in slice order by a second launch (N % 4 == 0)
   float* part;
   int kslices;
+  int split_rf;         // rows per tile / 32 of a split launch (qproj_split_plan)
   // optional: set to 1 when an fp16 conversion of this launch (the general
   // kernel's x tiles, the fast epilogue's yh) met a bf16 value of magnitude
   // >= 2^16, inf or NaN (see range_report)
@@ -269,6 +270,8 @@ hipError_t validate_gemv_kernels();
 // ---- the fast quantized route (qproj_fast.hip) --------------------------------
 // x is fp16 (carrying bf16 values), a.codes / a.sb the fast resident layout.
 hipError_t launch_qproj_fast(int bits, const QprojArgs& a, hipStream_t s);
+// K slices of a projection of few tiles, and its tile height (0: no split).
+int qproj_split_plan(int M, int N, int K, int* rf);
 // The gate and up projections of a SwiGLU in one launch (the fields after
 // `range` in QprojArgs): each 256 x 256 tile holds 128 columns of each, so
 // the gate's output meets the up projection's in LDS and only

@@ -11,19 +11,16 @@
 //     v_pk_fma_f16 on the exact integer code (built with the 0x6400 magic:
 //     (0x6400 | c) is 1024 + c in fp16, and 1024 is subtracted exactly).
 //
-// Per block: 256 threads (4 wave64s), tile 256(M) x 256(N) x 64(K); the
-// waves split N, each owning 64 columns x 256 rows (2 x 8 tiles of
-// v_mfma_f32_32x32x16_f16), so each weight is dequantized once. Per stage
-// the DMA moves the fp16 x tile (32 KB), the code tile (8 KB w4 / 16 KB
-// w8) and 256 fp16 (scale, bias) pairs. No VGPR round trip, and each wave
-// waits on its own vmcnt for the stage two behind the one in flight.
-// Every stage buffer is its own __shared__ object so the compiler's LDS-DMA
-// tracking sees that reads of one stage do not alias the DMA into another.
+// Per block: tile 32*RF(M) x 256(N) x 64(K). At 256 rows 4 wave64s split N,
+// each owning 64 columns x all rows (2 x 8 tiles of v_mfma_f32_32x32x16_f16),
+// so each weight is dequantized once; the lower tiles (kTiles) run 8 waves of
+// 32 columns. Per stage the DMA moves the fp16 x tile (32 KB at 256 rows), the
+// code tile (8 KB w4 / 16 KB w8) and 256 fp16 (scale, bias) pairs. No VGPR
+// round trip, and each wave waits on its own vmcnt for the stage two behind
+// the one in flight.
 //
 // The same body also runs as qproj_pair_kernel (a SwiGLU's gate and up
-// projections in one tile, 128 columns of each) and, for the last tile row
-// of a paired grid whose last round would hold only that row, with 128-row
-// tiles (4 row fragments a wave instead of 8).
+// projections in one tile, 128 columns of each), and split along K (few tiles).
 //
 // Resident code layout this kernel reads (built by repack_*_fast):
 //   w4: codes[kt][n][fk][kk]   one u32 = the 8 codes of k = 16kk + 8fk + 0..7,
@@ -102,36 +99,43 @@ __device__ __forceinline__ int wchunk(int n, int h) {
 // then sums the slices in order and finishes as the epilogue does.
 //
 // PAIR (launch_qproj_pair): the tile's 256 weight rows are 128 rows of the
-// gate weight (waves 0-1) and the same 128 rows of the up weight (waves
-// 2-3); the tail stages the gate's and the up projection's T chunks side by
+// gate weight (the first half of the waves) and the same 128 rows of the up
+// weight (the second half); the tail stages the gate's and the up projection's T chunks side by
 // side; the epilogue meets the two in LDS and writes only the SwiGLU.
-template <int BITS, bool SPLIT, bool PAIR, int RF>
+template <int BITS, bool SPLIT, bool PAIR, int RF, int NW>
 __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   constexpr int WCH = BITS == 4 ? 512 : 1024;    // 16-B code chunks per stage
   constexpr int CPR = BITS == 4 ? 2 : 4;         // code chunks per row
-  constexpr int WDMA = WCH / 256;                // code DMAs per wave per stage
+  constexpr int WDMA = WCH / (64 * NW);          // code DMAs per wave per stage
+  constexpr int JT = 8 / NW;                     // 32-column tiles per wave
   constexpr int BMT = 32 * RF;                   // rows per tile: RF fragments of 32
-  constexpr int XD = RF;                         // x DMAs per wave per stage
-  constexpr int TD = RF / 2;                     // T DMAs per wave per tail chunk
+  constexpr int XD = 4 * RF / NW;                // x DMAs per wave per stage
+  static_assert(XD * NW == 4 * RF, "x DMAs divide among the waves");
+  constexpr int TD = (2 * RF + NW - 1) / NW;     // T DMAs per wave per tail chunk
+  constexpr int BD = 16 / NW;                    // B DMAs per wave per tail chunk
   constexpr int PER = XD + WDMA + 1;             // DMAs per wave per base stage
-  constexpr int TPER = (PAIR ? 2 : 1) * TD + 4;  // DMAs per wave per tail chunk
+  constexpr int TPER = (PAIR ? 2 : 1) * TD + BD; // DMAs per wave per tail chunk
   constexpr int BNT = PAIR ? BN / 2 : BN;        // output columns per tile
-  // One __shared__ object per stage: [x 32 KB | codes | (s, b)]; a tail
-  // chunk is [T 16 KB | B 16 KB (| the up projection's T 16 KB)].
+  // A stage is [x tile | codes | (s, b)], a tail chunk [T | B (| the up
+  // projection's T)]; the epilogue takes four 16 KB regions.
+  constexpr int TRG = 64 * NW * TD;              // a tail chunk's T region
   constexpr int STG0 = BMT * 8 + WCH + BN / 4;
-  constexpr int STG = PAIR && STG0 < 3072 ? 3072 : STG0;
-  __shared__ uint4 st0[STG], st1[STG], st2[STG];
+  constexpr int TSTG = (PAIR ? 2 : 1) * TRG + 1024;
+  constexpr int STG = STG0 < TSTG ? TSTG : STG0;
+  __shared__ uint4 ring[3 * STG < 4096 ? 4096 : 3 * STG];
+  static_assert(3 * STG <= 10240, "the CU's 160 KB");
+  uint4 *const st0 = ring, *const st1 = ring + STG, *const st2 = ring + 2 * STG;
 
-  // Waves split N only: wave w owns output columns [64w, 64w+64) for all
-  // 256 rows (2 x 8 tiles of 32x32), so every weight fragment is
-  // dequantized by exactly one wave.
+  // Waves split N only: wave w owns the 32*JT output columns from 32*JT*w for
+  // all of the tile's rows, so every weight fragment is dequantized by exactly
+  // one wave.
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 31, fk = lane >> 5;
-  // PAIR: waves 2-3 read the up weight; their columns are the gate's again
-  const bool upw = PAIR && wave >= 2;
-  const int wcol = PAIR ? 64 * (wave & 1) : 64 * wave;
+  // PAIR: the second half of the waves reads the up weight; their columns are
+  // the gate's again
+  const bool upw = PAIR && wave >= NW / 2;
 
   const int tiles_m = (a.M + BMT - 1) / BMT;
   const int tiles_n = (a.N + BNT - 1) / BNT;
@@ -140,12 +144,24 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   if constexpr (SPLIT) {
     ks = blk / (tiles_m * tiles_n);
     blk -= ks * (tiles_m * tiles_n);
-    kt0 = KT * ks / a.kslices;
-    KT = KT * (ks + 1) / a.kslices - kt0;
   }
   tile_of_block(blk, tiles_m, tiles_n, &tm, &tn);
   const int m0 = tm * BMT, n0 = tn * BNT;
   const int mlast = a.M - 1, nlast = a.N - 1;
+  int sg = 0;                                    // the tile's segment
+  for (int i = 1; i < a.nseg; ++i)
+    if (n0 >= a.seg[i].n_begin) sg = i;
+  if constexpr (SPLIT) {
+    // the last slice also runs the LoRA tail, a chunk of it about 5/8 of a
+    // stage: it takes that much less of K (at least one stage each)
+    const int total = KT + a.seg[sg].chunks * 5 / 8;
+    auto bound = [&](int i) {
+      const int b = total * i / a.kslices, m = KT - (a.kslices - i);
+      return b < m ? b : m;
+    };
+    kt0 = bound(ks);
+    KT = bound(ks + 1) - kt0;
+  }
 
   // stage 0 of this block's K range
   const _Float16* __restrict__ x16 = reinterpret_cast<const _Float16*>(a.x) + (long long)kt0 * BK;
@@ -179,7 +195,10 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
     n = n < nlast ? n : nlast;
     woff[i] = (uint32_t)((n * CPR + h) * 16);
   }
-  int sn = n0 + wcol + lane;
+  // (s, b): 64 columns a wave from sst; with eight waves the runs overlap
+  // (the same values), never across the tile's halves
+  const int sst = NW == 4 ? 64 * wave : 128 * (wave >> 2) + (32 * (wave & 3) < 64 ? 32 * (wave & 3) : 64);
+  int sn = n0 + (PAIR ? sst & 127 : sst) + lane;
   sn = sn < nlast ? sn : nlast;
   const uint32_t soff = (uint32_t)sn * 4u;
 
@@ -189,7 +208,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
     if (g < 2) {
       const void* base = x16 + (long long)kt * BK;
 #pragma unroll
-      for (int i = (XD / 2) * g; i < (XD / 2) * (g + 1); ++i)
+      for (int i = g ? XD / 2 : 0; i < (g ? XD : XD / 2); ++i)
         dma16_sb(base, xoff[i], lds_addr(B + 64 * (XD * wave + i)));
     } else {
       const void* wbase = codes + (long long)kt * a.N * CPR;
@@ -197,13 +216,13 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
       for (int i = 0; i < WDMA; ++i)
         dma16_sb(wbase, woff[i], lds_addr(B + BMT * 8 + 64 * (WDMA * wave + i)));
       dma4_sb(sbp + (long long)kt * a.N, soff,
-              lds_addr(reinterpret_cast<const uint32_t*>(B + BMT * 8 + WCH) + 64 * wave));
+              lds_addr(reinterpret_cast<const uint32_t*>(B + BMT * 8 + WCH) + sst));
     }
   };
 
-  floatx16_t acc[2][RF];
+  floatx16_t acc[JT][RF];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < JT; ++j)
 #pragma unroll
     for (int i = 0; i < RF; ++i)
 #pragma unroll
@@ -211,17 +230,17 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
 
   // Stage state in registers: the code words and (s, b) of the wave's two
   // n-tiles, and the current k16 step's operands.
-  uint4 wc[2][CPR / 2];
-  half2v s2[2], b2[2];
-  uint4 wa[2], xb[RF];
+  uint4 wc[JT][CPR / 2];
+  half2v s2[JT], b2[JT];
+  uint4 wa[JT], xb[RF];
 
-  auto load_ws = [&](const uint4* B, uint4 (&wcv)[2][CPR / 2], half2v (&s2v)[2],
-                     half2v (&b2v)[2]) {
+  auto load_ws = [&](const uint4* B, uint4 (&wcv)[JT][CPR / 2], half2v (&s2v)[JT],
+                     half2v (&b2v)[JT]) {
     const uint4* W = B + BMT * 8;
     const uint32_t* S = reinterpret_cast<const uint32_t*>(B + BMT * 8 + WCH);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = 64 * wave + 32 * j + fr;
+    for (int j = 0; j < JT; ++j) {
+      const int n = 32 * JT * wave + 32 * j + fr;
 #pragma unroll
       for (int h = 0; h < CPR / 2; ++h)
         wcv[j][h] = W[wchunk<CPR>(n, fk * (CPR / 2) + h)];
@@ -230,8 +249,8 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
       b2v[j] = __builtin_bit_cast(half2v, __builtin_amdgcn_perm(sb, sb, 0x03020302u));
     }
   };
-  auto deq = [&](const uint4 (&wcv)[2][CPR / 2], const half2v (&s2v)[2],
-                 const half2v (&b2v)[2], int j, int kk) -> uint4 {
+  auto deq = [&](const uint4 (&wcv)[JT][CPR / 2], const half2v (&s2v)[JT],
+                 const half2v (&b2v)[JT], int j, int kk) -> uint4 {
     if constexpr (BITS == 4) {
       return deq_w4((&wcv[j][0].x)[kk], s2v[j], b2v[j]);
     } else {
@@ -255,30 +274,38 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
     const int nk = kt + 2 < KT ? kt + 2 : KT - 1;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
-      uint4 wn_[2], xn_[RF];
-      uint4 wcn[2][CPR / 2];
-      half2v s2n[2], b2n[2];
+      uint4 wn_[JT], xn_[RF];
+      uint4 wcn[JT][CPR / 2];
+      half2v s2n[JT], b2n[JT];
       if (kk < 3) {
         issue_grp(kk, nk, Pv);
 #pragma unroll
         for (int i = 0; i < RF; ++i) xn_[i] = C[swz8(32 * i + fr, 2 * (kk + 1) + fk)];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) wn_[j] = deq(wc, s2, b2, j, kk + 1);
+        for (int j = 0; j < JT; ++j) wn_[j] = deq(wc, s2, b2, j, kk + 1);
       } else {
         load_ws(Nx, wcn, s2n, b2n);
 #pragma unroll
         for (int i = 0; i < RF; ++i) xn_[i] = Nx[swz8(32 * i + fr, fk)];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) wn_[j] = deq(wcn, s2n, b2n, j, 0);
+        for (int j = 0; j < JT; ++j) wn_[j] = deq(wcn, s2n, b2n, j, 0);
       }
 #pragma unroll
       for (int i = 0; i < RF; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < JT; ++j)
           acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
               __builtin_bit_cast(half8_t, wa[j]), __builtin_bit_cast(half8_t, xb[i]),
               acc[j][i], 0, 0, 0);
-      if (kk < 3) {
+      if constexpr (NW == 8) {
+        // two waves a SIMD: only the reads are pinned ahead of the MFMAs
+#pragma unroll
+        for (int g = 0; g < RF; ++g) {
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 16 / RF, 0);
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+      } else if (kk < 3) {
 #pragma unroll
         for (int g = 0; g < RF; ++g) {
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // DS read
@@ -286,27 +313,27 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
         }
 #pragma unroll
         for (int g = 0; g < RF; ++g) {
-          __builtin_amdgcn_sched_group_barrier(0x002, 32 / RF, 0);   // VALU
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);         // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x002, (32 + RF - 1) / RF, 0);   // VALU
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                    // MFMA
         }
       } else {
         // step 3: NDS reads over the DSM MFMAs left after the VG that carry
         // the next stage's first dequantization (w4 at 256 rows: spread
         // over 10 MFMAs, 4 VALU each, which measured ~0.5% faster launches
         // than 6 MFMAs of 6; the reads then go two per MFMA)
-        constexpr int NDS = RF + 2 * (CPR / 2) + 2;
+        constexpr int NDS = RF + JT * (CPR / 2) + JT;
         constexpr int VG = RF == 8 && CPR == 2 ? RF + 2 : 3 * RF / 4;
         constexpr int VPG = RF == 8 && CPR == 2 ? 4 : 6;   // VALU per group
         constexpr int DSM = 2 * RF - VG;
-        static_assert(NDS >= DSM && NDS <= 2 * DSM, "step-3 DS reads per MFMA pin");
+        constexpr int DPM = NDS / DSM, XTRA = NDS - DPM * DSM;   // reads per MFMA
 #pragma unroll
-        for (int g = 0; g < NDS - DSM; ++g) {
-          __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        for (int g = 0; g < XTRA; ++g) {
+          __builtin_amdgcn_sched_group_barrier(0x100, DPM + 1, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
 #pragma unroll
-        for (int g = NDS - DSM; g < DSM; ++g) {
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        for (int g = XTRA; g < DSM; ++g) {
+          __builtin_amdgcn_sched_group_barrier(0x100, DPM, 0);
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
 #pragma unroll
@@ -321,12 +348,12 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) wa[j] = wn_[j];
+      for (int j = 0; j < JT; ++j) wa[j] = wn_[j];
 #pragma unroll
       for (int i = 0; i < RF; ++i) xb[i] = xn_[i];
       if (kk == 3) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < JT; ++j) {
 #pragma unroll
           for (int h = 0; h < CPR / 2; ++h) wc[j][h] = wcn[j][h];
           s2[j] = s2n[j];
@@ -346,7 +373,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
 #pragma unroll
   for (int i = 0; i < RF; ++i) xb[i] = st0[swz8(32 * i + fr, fk)];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) wa[j] = deq(wc, s2, b2, j, 0);
+  for (int j = 0; j < JT; ++j) wa[j] = deq(wc, s2, b2, j, 0);
 
   // Stage kt lives in buffer kt % 3; three stages per trip, the remainder
   // (KT % 3) after the loop, so the loop body has no branch.
@@ -361,12 +388,9 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   ring_wait<0>();                               // drained; LDS free
 
   // ---- LoRA tail: T and gathered B chunks of 32 ranks, same ring ----
-  int sg = 0;
-  for (int i = 1; i < a.nseg; ++i)
-    if (n0 >= a.seg[i].n_begin) sg = i;
   const int chunks32 = (!SPLIT || ks == a.kslices - 1) ? a.seg[sg].chunks : 0;
   if (chunks32 > 0) {
-    // PAIR: waves 2-3 gather the up projection's B (its segment, its
+    // PAIR: the second half of the waves gathers the up projection's B (its segment, its
     // groups); both T chunks are staged for every wave
     const QprojSeg& sw = upw ? a.seg_u : a.seg[sg];
     const int t_col0 = a.seg[sg].t_col0;
@@ -378,14 +402,15 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
     // the first live group of the segment: a finite source for padding
     // groups (their T columns are exactly 0)
     const int g_safe = a.grp[grp0];
-    // T: BMT rows x 4 chunks (TD DMAs a wave); B: 256 rows x 4 chunks (4)
+    // T: BMT rows x 4 chunks (TD DMAs a wave, rounded up: rows past the tile
+    // land in the region's end, unread); B: 256 rows x 4 chunks (BD)
     uint32_t toff[TD];
-    uint32_t boff[4];
-    int bc[4];
-    if constexpr (TD == 4) {
+    uint32_t boff[BD];
+    int bc[BD];
+    if constexpr (TD == BD) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int p = 64 * (4 * wave + i) + lane;
+      for (int i = 0; i < BD; ++i) {
+        const int p = 64 * (BD * wave + i) + lane;
         const int row = p >> 2;
         const int c = (p & 3) ^ ((row >> 2) & 3);
         int m = m0 + row;
@@ -407,8 +432,8 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
         toff[i] = (uint32_t)(((long long)m * a.ldt + t_col0 + 8 * c) * 2);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int p = 64 * (4 * wave + i) + lane;
+      for (int i = 0; i < BD; ++i) {
+        const int p = 64 * (BD * wave + i) + lane;
         const int row = p >> 2;
         const int c = (p & 3) ^ ((row >> 2) & 3);
         int n = n0 + (PAIR ? (row & 127) : row);
@@ -417,8 +442,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
         bc[i] = c;
       }
     }
-    // T region = first 16 KB of the stage buffer, B region = second. A
-    // lane's 16 bytes are the 8 ranks of one group; the chunk's four groups
+    // A lane's 16 bytes are the 8 ranks of one group; the chunk's four groups
     // are wave-uniform (scalar loads).
     auto grp_word = [&](int ch) -> uint2 {
       const int gi = __builtin_amdgcn_readfirstlane(grp0 + 4 * ch);
@@ -432,7 +456,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
       if constexpr (PAIR) {
 #pragma unroll
         for (int i = 0; i < TD; ++i)
-          dma16_sb(tu + 32 * ch, toff[i], lds_addr(X + 2048 + 64 * (TD * wave + i)));
+          dma16_sb(tu + 32 * ch, toff[i], lds_addr(X + TRG + 1024 + 64 * (TD * wave + i)));
       }
       // The chunk's four groups are one aligned 8-byte word of the table (a
       // segment's groups start at a multiple of 4), read by a wave-uniform
@@ -442,19 +466,19 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
       const int nx = ch + 1 < chunks32 ? ch + 1 : chunks32 - 1;
       gw_next = grp_word(nx);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < BD; ++i) {
         const uint32_t w = (bc[i] & 2) ? gw.y : gw.x;
         int g = (int16_t)(w >> ((bc[i] & 1) << 4));
         g = g < 0 ? g_safe : g;
-        dma16_sb(Bp, boff[i] + (uint32_t)g * 16u, lds_addr(X + 1024 + 64 * (4 * wave + i)));
+        dma16_sb(Bp, boff[i] + (uint32_t)g * 16u, lds_addr(X + TRG + 64 * (BD * wave + i)));
       }
     };
-    uint4 ta[2], tb[RF];
-    auto read_t = [&](const uint4* X, int kk, uint4 (&av)[2], uint4 (&bv)[RF]) {
+    uint4 ta[JT], tb[RF];
+    auto read_t = [&](const uint4* X, int kk, uint4 (&av)[JT], uint4 (&bv)[RF]) {
       const int c = 2 * kk + fk;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) av[j] = X[1024 + swz4(64 * wave + 32 * j + fr, c)];
-      const uint4* const XT = upw ? X + 2048 : X;
+      for (int j = 0; j < JT; ++j) av[j] = X[TRG + swz4(32 * JT * wave + 32 * j + fr, c)];
+      const uint4* const XT = upw ? X + TRG + 1024 : X;
 #pragma unroll
       for (int i = 0; i < RF; ++i) bv[i] = XT[swz4(32 * i + fr, c)];
     };
@@ -465,7 +489,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
       const int nc = ch + 2 < chunks32 ? ch + 2 : chunks32 - 1;
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
-        uint4 an[2], bn[RF];
+        uint4 an[JT], bn[RF];
         if (kk == 0) {
           issue_t(nc, Pv);
           read_t(C, 1, an, bn);
@@ -475,13 +499,13 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
 #pragma unroll
         for (int i = 0; i < RF; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
+          for (int j = 0; j < JT; ++j)
             acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                 __builtin_bit_cast(bf16x8_t, ta[j]), __builtin_bit_cast(bf16x8_t, tb[i]),
                 acc[j][i], 0, 0, 0);
 #pragma unroll
-        for (int g = 0; g < 2 + RF; ++g) {
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // DS read
+        for (int g = 0; g < (JT + RF < JT * RF ? JT + RF : JT * RF); ++g) {
+          __builtin_amdgcn_sched_group_barrier(0x100, JT + RF <= JT * RF ? 1 : 2, 0);   // DS read
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -490,7 +514,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
           __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int j = 0; j < 2; ++j) ta[j] = an[j];
+        for (int j = 0; j < JT; ++j) ta[j] = an[j];
 #pragma unroll
         for (int i = 0; i < RF; ++i) tb[i] = bn[i];
       }
@@ -517,10 +541,10 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
       const int m = m0 + 32 * i + fr;
       if (m >= a.M) continue;
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < JT; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int n = n0 + 64 * wave + 32 * j + 8 * q + 4 * fk;
+          const int n = n0 + 32 * JT * wave + 32 * j + 8 * q + 4 * fk;
           if (n < a.N)
             *reinterpret_cast<float4*>(a.part + ((long long)ks * a.M + m) * a.N + n) =
                 make_float4(acc[j][i][4 * q + 0], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2],
@@ -537,23 +561,24 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
     // [64 (w >> 1), +64) from the gate's region c and the up projection's
     // region 2 + c, and writes y = bf16(silu(g) * u) and its fp16 copy: the
     // bits of the gate's own epilogue followed by the gated one.
-    uint2* const Ew = reinterpret_cast<uint2*>((wave < 2 ? st0 : st1) + 1024 * (wave & 1));
-    const uint4* const Eg = st0 + 1024 * (wave & 1);
-    const uint4* const Eu = st1 + 1024 * (wave & 1);
+    const int rg = wave * JT / 2;   // the 64-column region this wave writes
+    uint2* const Ew = reinterpret_cast<uint2*>(ring + 1024 * rg);
+    const uint4* const Eg = ring + 1024 * (wave & 1);
+    const uint4* const Eu = ring + 2048 + 1024 * (wave & 1);
     const int cl = lane & 7;
-    const int n = n0 + wcol + 8 * cl;
+    const int n = n0 + 64 * (wave & 1) + 8 * cl;
     uint32_t seen = 0;
 #pragma unroll
-    for (int h = 0; h < RF / 4; ++h) {
+    for (int h = 0; h < (RF + 3) / 4; ++h) {
 #pragma unroll
-      for (int ii = 0; ii < 4; ++ii) {
+      for (int ii = 0; ii < (RF - 4 * h < 4 ? RF - 4 * h : 4); ++ii) {
         const int i = 4 * h + ii;
         const int ml = 32 * ii + fr;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < JT; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const int c = 4 * j + q;
+            const int c = 4 * (JT == 2 ? j : (wave & 1)) + q;
             uint2 v;
             v.x = pack_bf16x2_rne(acc[j][i][4 * q + 0], acc[j][i][4 * q + 1]);
             v.y = pack_bf16x2_rne(acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]);
@@ -562,8 +587,8 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
       }
       __syncthreads();
 #pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const int ml = 64 * (wave >> 1) + 8 * r + (lane >> 3);
+      for (int r = 0; r < JT * (RF - 4 * h < 4 ? RF - 4 * h : 4); ++r) {
+        const int ml = 8 * JT * (RF - 4 * h < 4 ? RF - 4 * h : 4) * (wave >> 1) + 8 * r + (lane >> 3);
         const int e = ml * 8 + (cl ^ ((ml >> 1) & 7));
         const uint4 gv = Eg[e];
         uint4 v = Eu[e];
@@ -599,20 +624,22 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   // conflict-free), then stores whole 128-B row segments, 8 rows per
   // instruction. Only the wave itself touches its region, and LDS accesses
   // of one wave complete in order, so no barrier is needed inside.
-  uint4* const E = (wave < 2 ? st0 : st1) + 1024 * (wave & 1);
+  const int rg = wave * JT / 2;   // the 64-column region this wave writes and stores from
+  uint4* const E = ring + 1024 * rg;
   const bool st16 = (a.ldy & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
   const int cl = lane & 7;
-  const int n = n0 + 64 * wave + 8 * cl;
+  const int n = n0 + 64 * rg + 8 * cl;
   uint32_t seen = 0;   // magnitudes written to the fp16 copy (range_report)
 #pragma unroll
-  for (int h = 0; h < RF / 4; ++h) {
+  for (int h = 0; h < (RF + 3) / 4; ++h) {
+    const int HF = RF - 4 * h < 4 ? RF - 4 * h : 4;   // fragments of this part
     // Fused SwiGLU: this half's gate rows are loaded first, so their memory
     // latency overlaps the conversion below instead of stalling each store.
     uint4 gv[16];
     if (a.g) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        int m = m0 + 128 * h + 8 * r + (lane >> 3);
+      for (int r = 0; r < 2 * JT * HF; ++r) {
+        int m = m0 + 128 * h + (JT == 2 ? 0 : 16 * HF * (wave & 1)) + 8 * r + (lane >> 3);
         m = m < a.M ? m : a.M - 1;
         const int nn = n < a.N ? n : a.N - 8;
         gv[r] = *reinterpret_cast<const uint4*>(a.g + (long long)m * a.ldg + nn);
@@ -620,23 +647,26 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
     }
     uint2* const E2 = reinterpret_cast<uint2*>(E);
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
+    for (int ii = 0; ii < HF; ++ii) {
       const int i = 4 * h + ii;
       const int ml = 32 * ii + fr;
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < JT; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int c = 4 * j + q;
+          const int c = 4 * (JT == 2 ? j : (wave & 1)) + q;
           uint2 v;
           v.x = pack_bf16x2_rne(acc[j][i][4 * q + 0], acc[j][i][4 * q + 1]);
           v.y = pack_bf16x2_rne(acc[j][i][4 * q + 2], acc[j][i][4 * q + 3]);
           E2[ml * 16 + 2 * (c ^ ((ml >> 1) & 7)) + fk] = v;
         }
     }
+    // eight waves: two share a region, each writes its 32 columns and stores
+    // half of the rows
+    if constexpr (NW == 8) __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int ml = 8 * r + (lane >> 3);
+    for (int r = 0; r < 2 * JT * HF; ++r) {
+      const int ml = (JT == 2 ? 0 : 16 * HF * (wave & 1)) + 8 * r + (lane >> 3);
       uint4 v = E[ml * 8 + (cl ^ ((ml >> 1) & 7))];
       const int m = m0 + 128 * h + ml;
       if (m < a.M && n < a.N) {
@@ -667,20 +697,19 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
         }
       }
     }
+    if constexpr (NW == 8 && RF > 4) __syncthreads();
   }
   if (a.yh) range_report(a.range, seen);
 }
 
-template <int BITS, bool SPLIT>
-__global__ __launch_bounds__(256, 1) void qproj_fast_kernel(const QprojArgs a) {
-  qproj_fast_body<BITS, SPLIT, false, 8>(a);
+template <int BITS, bool SPLIT, int RF, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void qproj_fast_kernel(const QprojArgs a) {
+  qproj_fast_body<BITS, SPLIT, false, RF, NW>(a);
 }
 
-// RF = 8: 256-row tiles; RF = 4: 128-row tiles (the rows of a grid's last,
-// mostly empty round, see launch_qproj_pair)
-template <int BITS, int RF>
-__global__ __launch_bounds__(256, 1) void qproj_pair_kernel(const QprojArgs a) {
-  qproj_fast_body<BITS, false, true, RF>(a);
+template <int BITS, int RF, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void qproj_pair_kernel(const QprojArgs a) {
+  qproj_fast_body<BITS, false, true, RF, NW>(a);
 }
 
 // The split projection's end: y = bf16(sum of the slices in order), then as
@@ -1105,35 +1134,6 @@ __global__ void bf16_to_f16_kernel(const uint16_t* x, long long ldx, uint16_t* y
 
 }  // namespace
 
-hipError_t launch_qproj_fast(int bits, const QprojArgs& a, hipStream_t s) {
-  const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-  if (tiles <= 0) return hipSuccess;
-  if (a.kslices > 1) {
-    if (!a.part || a.N % 4 != 0 || (long long)a.M * (a.N / 4) >= (1ll << 31))
-      return hipErrorInvalidValue;
-    const dim3 grid((unsigned)(tiles * a.kslices));
-    if (bits == 4)
-      hipLaunchKernelGGL((qproj_fast_kernel<4, true>), grid, dim3(256), 0, s, a);
-    else if (bits == 8)
-      hipLaunchKernelGGL((qproj_fast_kernel<8, true>), grid, dim3(256), 0, s, a);
-    else
-      return hipErrorInvalidValue;
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    long long blocks = ((long long)a.M * (a.N / 4) + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(qproj_split_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
-    return hipGetLastError();
-  }
-  if (bits == 4)
-    hipLaunchKernelGGL((qproj_fast_kernel<4, false>), dim3(tiles), dim3(256), 0, s, a);
-  else if (bits == 8)
-    hipLaunchKernelGGL((qproj_fast_kernel<8, false>), dim3(tiles), dim3(256), 0, s, a);
-  else
-    return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
 // CUs of the current device (the launch rounds are counted against it).
 static int device_cus() {
   static int cached[64] = {};
@@ -1149,56 +1149,190 @@ static int device_cus() {
   return cached[dev];
 }
 
-// A grid whose last round of the chip's CUs is mostly empty (4352 rows: 1360
-// tiles, 80 in a sixth round on 256 CUs) runs its last tile row as 128-row
-// tiles in a second launch over the same arguments shifted down: twice the
-// blocks at about half the time each. Each output element
-// is computed by the same MFMA sequence either way, so the bits do not
-// depend on the split.
+// Rows per tile. A tile of 32*rf rows over 60 K stages takes, in one round of
+// the chip, about 35.5, 45, 56 and 73.5 us at rf 2, 4, 6 and 8 (w4, [M, 3840] x
+// [3840, 3840], M = 300..1493; other K in proportion): rf 8 is the best rate
+// for a full chip (1.15x the MFMA time), the lower tiles fill it where 256
+// rows leave it idle (1280 rows: 75 tiles, 75.5 -> 49.8 us with 150 of rf 4).
+// rf 2 to 6 run eight waves, two a SIMD, each 32 columns: 49.8 against 53.2 us
+// with four waves at rf 4; at rf 8 their reads of x would fill the LDS.
+struct TileCost {
+  int rf;
+  double us;
+};
+constexpr TileCost kTiles[4] = {{8, 73.5}, {6, 56.0}, {4, 45.0}, {2, 35.5}};
+
+// The rows of a launch: the first rows_main as 256-row tiles, the others as
+// tiles of rf_rest. Each output element is computed by the same MFMA sequence
+// in every tile height, so the bits do not depend on the plan.
+struct RowPlan {
+  int rows_main, rf_rest;
+};
+
+// Least time in rounds of the chip, one tile a CU, over whole rounds of
+// 256-row tiles followed by one of the heights (a second launch costs about
+// 3 us). 4352 rows of a paired launch (80 column tiles): 16 tile rows in five
+// rounds, then 256 rows as rf 4 in one.
+static RowPlan plan_rows(int M, int tiles_n, int rf_min) {
+  const int cus = device_cus();
+  const int tiles_m = (M + BM - 1) / BM;
+  auto rounds = [&](long long rows_of_tiles) {
+    return (double)((rows_of_tiles * tiles_n + cus - 1) / cus);
+  };
+  RowPlan best = {M, 8};
+  double cost = rounds(tiles_m) * kTiles[0].us;
+  const int all = (int)rounds(tiles_m);
+  for (int k = 0; k < 4; ++k) {
+    // the tile rows that fill all - 1 - k rounds (k = 3: none)
+    const long long full = k < 3 ? (long long)(all - 1 - k) * cus / tiles_n : 0;
+    const int m1 = full < 0 ? 0 : full < tiles_m ? (int)full : tiles_m - 1;
+    const double head = m1 > 0 ? rounds(m1) * kTiles[0].us + 3.0 : 0.0;
+    for (const TileCost& t : kTiles) {
+      if (t.rf < rf_min) continue;
+      const double c = head + rounds((M - m1 * BM + 32 * t.rf - 1) / (32 * t.rf)) * t.us;
+      if (c < cost) {
+        cost = c;
+        best = {m1 * BM, t.rf};
+      }
+    }
+  }
+  return best;
+}
+
+// The K split of a projection of few 256 x 256 tiles (the context refiner's
+// caption rows: 15 or 40): rows per tile and slices, by the time of a round
+// (a stage of 64 about 0.45, 0.57 and 0.96 us at rf 2, 4 and 8) plus the f32
+// partials, written and read at about 5 TB/s. Never more slices than 256-row
+// tiles would take (one round, at least 6 stages each), so the partials stay
+// within what they would take. [256, 3840] x [3840, 3840]: rf 2 in 4 slices, 24.6
+// us, where rf 8 in 10 took 30.7; 16 rows 14.1 against 18.6. 0: no split.
+int qproj_split_plan(int M, int N, int K, int* rf) {
+  *rf = 8;
+  const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  if (tiles <= 0 || tiles >= 64 || N % 4 != 0) return 0;
+  const int KT = K / BK;
+  int kmax = 256 / tiles;
+  if (kmax > KT / 6) kmax = KT / 6;
+  if (kmax < 2) return 0;
+  const int cus = device_cus();
+  const TileCost stage[3] = {{8, 0.96}, {4, 0.57}, {2, 0.45}};
+  int best = 0;
+  double cost = 0.0;
+  for (const TileCost& t : stage) {
+    const int grid = ((M + 32 * t.rf - 1) / (32 * t.rf)) * ((N + BN - 1) / BN);
+    for (int ks = 2; ks <= kmax; ++ks) {
+      const double c = (double)((grid * ks + cus - 1) / cus) * ((KT + ks - 1) / ks) * t.us +
+                       1.6e-6 * (double)M * N * ks;
+      if (best == 0 || c < cost) {
+        cost = c;
+        best = ks;
+        *rf = t.rf;
+      }
+    }
+  }
+  return best;
+}
+
+template <int BITS, bool SPLIT, int RF, int NW>
+static void launch_tiles(const QprojArgs& a, hipStream_t s) {
+  const int tiles = ((a.M + 32 * RF - 1) / (32 * RF)) * ((a.N + BN - 1) / BN);
+  hipLaunchKernelGGL((qproj_fast_kernel<BITS, SPLIT, RF, NW>),
+                     dim3((unsigned)(SPLIT ? tiles * a.kslices : tiles)), dim3(64 * NW), 0, s, a);
+}
+template <int BITS>
+static void launch_rows(const QprojArgs& a, int rf, hipStream_t s) {
+  switch (rf) {
+    case 2: launch_tiles<BITS, false, 2, 8>(a, s); break;
+    case 4: launch_tiles<BITS, false, 4, 8>(a, s); break;
+    case 6: launch_tiles<BITS, false, 6, 8>(a, s); break;
+    default: launch_tiles<BITS, false, 8, 4>(a, s); break;
+  }
+}
+template <int BITS>
+static void launch_split(const QprojArgs& a, hipStream_t s) {
+  switch (a.split_rf) {
+    case 2: launch_tiles<BITS, true, 2, 8>(a, s); break;
+    case 4: launch_tiles<BITS, true, 4, 8>(a, s); break;
+    default: launch_tiles<BITS, true, 8, 4>(a, s); break;
+  }
+}
+template <int BITS, int RF, int NW>
+static void launch_pair_tiles(const QprojArgs& a, hipStream_t s) {
+  const int tiles = ((a.M + 32 * RF - 1) / (32 * RF)) * ((a.N + BN / 2 - 1) / (BN / 2));
+  hipLaunchKernelGGL((qproj_pair_kernel<BITS, RF, NW>), dim3((unsigned)tiles), dim3(64 * NW), 0,
+                     s, a);
+}
+template <int BITS>
+static void launch_pair_rows(const QprojArgs& a, int rf, hipStream_t s) {
+  switch (rf) {
+    case 4: launch_pair_tiles<BITS, 4, 8>(a, s); break;
+    case 6: launch_pair_tiles<BITS, 6, 8>(a, s); break;
+    default: launch_pair_tiles<BITS, 8, 4>(a, s); break;
+  }
+}
+
+// `rows(args, rf)` over the plan's two row ranges (the second one's arguments
+// shifted down by the first's rows).
+template <class F>
+static hipError_t launch_plan(const QprojArgs& a, const RowPlan& p, F&& rows) {
+  if (p.rows_main > 0) {
+    QprojArgs m = a;
+    m.M = p.rows_main;
+    rows(m, 8);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || p.rows_main == a.M) return e;
+  }
+  QprojArgs h = a;
+  const long long r = p.rows_main;
+  h.M = a.M - p.rows_main;
+  h.x = a.x + r * a.ldx;
+  h.y = a.y + r * a.ldy;
+  if (a.g) h.g = a.g + r * a.ldg;
+  if (a.yh) h.yh = a.yh + r * a.ldyh;
+  if (a.t) h.t = a.t + r * a.ldt;
+  rows(h, p.rf_rest);
+  return hipGetLastError();
+}
+
+hipError_t launch_qproj_fast(int bits, const QprojArgs& a, hipStream_t s) {
+  if (a.M <= 0 || a.N <= 0) return hipSuccess;
+  if (bits != 4 && bits != 8) return hipErrorInvalidValue;
+  if (a.kslices > 1) {
+    if (!a.part || a.N % 4 != 0 || (long long)a.M * (a.N / 4) >= (1ll << 31) ||
+        a.K / BK < a.kslices)
+      return hipErrorInvalidValue;
+    if (bits == 4)
+      launch_split<4>(a, s);
+    else
+      launch_split<8>(a, s);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    long long blocks = ((long long)a.M * (a.N / 4) + 255) / 256;
+    if (blocks > 4096) blocks = 4096;
+    hipLaunchKernelGGL(qproj_split_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
+    return hipGetLastError();
+  }
+  return launch_plan(a, plan_rows(a.M, (a.N + BN - 1) / BN, 2), [&](const QprojArgs& m, int rf) {
+    if (bits == 4)
+      launch_rows<4>(m, rf, s);
+    else
+      launch_rows<8>(m, rf, s);
+  });
+}
+
 hipError_t launch_qproj_pair(int bits, const QprojArgs& a, hipStream_t s) {
-  const int tiles_n = (a.N + BN / 2 - 1) / (BN / 2);
-  const int tiles_m = (a.M + BM - 1) / BM;
-  const int tiles = tiles_m * tiles_n;
-  if (tiles <= 0) return hipSuccess;
+  if (a.M <= 0 || a.N <= 0) return hipSuccess;
   if (a.kslices > 1 || a.g || !a.codes_u || !a.sb_u || a.nseg != 1 ||
       a.seg[0].chunks != a.seg_u.chunks || a.N % 8 != 0 || a.ldy % 8 != 0 ||
       (reinterpret_cast<uintptr_t>(a.y) & 15) != 0 || (bits != 4 && bits != 8))
     return hipErrorInvalidValue;
-  // Rounds of the chip, one 256-row tile a CU: the whole grid against the
-  // grid without its last tile row plus that row as 128-row tiles (about
-  // 0.55 of a round each, measured); split when that saves a fifth of a
-  // round or more.
-  const int cus = device_cus();
-  const int main_tiles = tiles - tiles_n;
-  const int half_blocks = ((a.M - (tiles_m - 1) * BM + BM / 2 - 1) / (BM / 2)) * tiles_n;
-  const double rounds_whole = (double)((tiles + cus - 1) / cus);
-  const double rounds_split =
-      (double)((main_tiles + cus - 1) / cus) + 0.55 * (double)((half_blocks + cus - 1) / cus);
-  const int rows_main =
-      (tiles_m >= 2 && rounds_split + 0.2 <= rounds_whole) ? (tiles_m - 1) * BM : a.M;
-  {
-    QprojArgs m = a;
-    m.M = rows_main;
-    const dim3 grid((unsigned)(tiles_m - (rows_main < a.M ? 1 : 0)) * tiles_n);
-    if (bits == 4)
-      hipLaunchKernelGGL((qproj_pair_kernel<4, 8>), grid, dim3(256), 0, s, m);
-    else
-      hipLaunchKernelGGL((qproj_pair_kernel<8, 8>), grid, dim3(256), 0, s, m);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || rows_main == a.M) return e;
-  }
-  QprojArgs h = a;
-  h.M = a.M - rows_main;
-  h.x = a.x + (long long)rows_main * a.ldx;
-  h.y = a.y + (long long)rows_main * a.ldy;
-  if (a.yh) h.yh = a.yh + (long long)rows_main * a.ldyh;
-  if (a.t) h.t = a.t + (long long)rows_main * a.ldt;
-  const dim3 grid((unsigned)(((h.M + BM / 2 - 1) / (BM / 2)) * tiles_n));
-  if (bits == 4)
-    hipLaunchKernelGGL((qproj_pair_kernel<4, 4>), grid, dim3(256), 0, s, h);
-  else
-    hipLaunchKernelGGL((qproj_pair_kernel<8, 4>), grid, dim3(256), 0, s, h);
-  return hipGetLastError();
+  return launch_plan(a, plan_rows(a.M, (a.N + BN / 2 - 1) / (BN / 2), 4),
+                     [&](const QprojArgs& m, int rf) {
+                       if (bits == 4)
+                         launch_pair_rows<4>(m, rf, s);
+                       else
+                         launch_pair_rows<8>(m, rf, s);
+                     });
 }
 
 // The K split depends on M and K only, never on how many columns are
@@ -1284,18 +1418,30 @@ hipError_t launch_bf16_to_f16(const uint16_t* x, long long ldx, uint16_t* y,
 
 hipError_t validate_qproj_fast_kernels() {
   hipFuncAttributes fa;
-  const void* fns[] = {reinterpret_cast<const void*>(&qproj_fast_kernel<4, false>),
-                       reinterpret_cast<const void*>(&qproj_fast_kernel<8, false>),
-                       reinterpret_cast<const void*>(&qproj_fast_kernel<4, true>),
-                       reinterpret_cast<const void*>(&qproj_fast_kernel<8, true>),
+  const void* fns[] = {reinterpret_cast<const void*>(&qproj_fast_kernel<4, false, 2, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<4, false, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<4, false, 6, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<4, false, 8, 4>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<4, true, 2, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<4, true, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<4, true, 8, 4>),
+                       reinterpret_cast<const void*>(&qproj_pair_kernel<4, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_pair_kernel<4, 6, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<8, false, 2, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<8, false, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<8, false, 6, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<8, false, 8, 4>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<8, true, 2, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<8, true, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_fast_kernel<8, true, 8, 4>),
+                       reinterpret_cast<const void*>(&qproj_pair_kernel<8, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_pair_kernel<8, 6, 8>),
                        reinterpret_cast<const void*>(&qproj_split_reduce_kernel),
                        reinterpret_cast<const void*>(&repack_fast_kernel),
                        reinterpret_cast<const void*>(&repack_sbf_kernel),
                        reinterpret_cast<const void*>(&bf16_to_f16_kernel),
-                       reinterpret_cast<const void*>(&qproj_pair_kernel<4, 8>),
-                       reinterpret_cast<const void*>(&qproj_pair_kernel<8, 8>),
-                       reinterpret_cast<const void*>(&qproj_pair_kernel<4, 4>),
-                       reinterpret_cast<const void*>(&qproj_pair_kernel<8, 4>),
+                       reinterpret_cast<const void*>(&qproj_pair_kernel<4, 8, 4>),
+                       reinterpret_cast<const void*>(&qproj_pair_kernel<8, 8, 4>),
                        reinterpret_cast<const void*>(&lora_xa_fast_kernel),
                        reinterpret_cast<const void*>(&lora_xa_reduce_kernel)};
   for (const void* f : fns) {

@@ -1022,9 +1022,7 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
               (uint64_t)M * (uint64_t)K * 2 <= (1ull << 31);
     any_fast = any_fast || fast[i];
   }
-  // Per projection: the fast route's K split on few tiles (the context
-  // refiner's 256 caption rows: 15 or 40 tiles), about one round of the
-  // chip at >= 6 K steps a slice; a dense weight with no live adapter on few
+  // Per projection: the fast route's K split on few tiles; a dense weight with no live adapter on few
   // 256 x 256 tiles (the caption embedder: 15; the final layer's 64
   // columns: 16) runs as the x.A path's split-K bf16 GEMM (identity column
   // groups, coefficient 1) where that is the faster one; it and the general
@@ -1040,13 +1038,9 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
     const ming_qweight* q = qs[i];
     const LinOut& o = outs[i];
     const int tiles = ((M + 255) / 256) * ((q->N + 255) / 256);
-    if (fast[i] && tiles < 64 && c->route == MING_ROUTE_AUTO && q->N % 4 == 0) {
-      int ks = 256 / tiles;
-      if (ks > (K / 64) / 6) ks = (K / 64) / 6;
-      if (ks >= 2) {
-        split_ks[i] = ks;
-        part_bytes = std::max(part_bytes, (size_t)ks * M * q->N * 4);
-      }
+    if (fast[i]) {
+      split_ks[i] = ming::qproj_split_plan(M, q->N, K, &qa[i].split_rf);
+      if (split_ks[i] >= 2) part_bytes = std::max(part_bytes, (size_t)split_ks[i] * M * q->N * 4);
     }
     const bool dense = q->bits == 16 && c->route != MING_ROUTE_GENERAL &&
                        (uint64_t)M * (uint64_t)ldx * 2 <= (1ull << 31) &&
