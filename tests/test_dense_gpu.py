@@ -82,3 +82,24 @@ def test_dense_gated_few_tiles(ctx, M):
     sync()
     assert np.array_equal(from_dev(got), from_dev(want))
     qw.close()
+
+
+# Tiles of 64 x 64 to 256 x 128, one slice and several, more columns than the
+# adapters' group table holds.
+@pytest.mark.parametrize("M,N,K", [(9, 4160, 1024), (17, 256, 4096), (130, 1984, 640),
+                                   (231, 1024, 2560), (300, 3840, 1024), (500, 704, 6400)])
+def test_dense_few_tiles(ctx, orc, M, N, K):
+    print(f"case dense split M={M} N={N} K={K}", flush=True)
+    x = bf16(randn(9800 + M, (M, K)))
+    pack, w = make_weight(9801 + N, N, K, 16, std=1.0 / np.sqrt(K))
+    b = bf16(randn(9802, (N,)))
+    qw = m.QWeight.dense(ctx, pack["w"])
+    xd, bd = to_dev(x), to_dev(b)
+    ref = orc.proj(x, w)
+    plain = _run(ctx, "auto", lambda y: ctx.lin(qw, xd, y, M), M, N)
+    biased = _run(ctx, "auto", lambda y: ctx.lin_bias(qw, xd, y, M, bd), M, N)
+    assert orc.rel_l2(orc.bf16_to_f32(plain), ref) <= TOL
+    assert orc.rel_l2(orc.bf16_to_f32(biased), ref + orc.bf16_to_f32(b)[None]) <= TOL
+    # slices are summed in order: the same bits again
+    assert np.array_equal(plain, _run(ctx, "auto", lambda y: ctx.lin(qw, xd, y, M), M, N))
+    qw.close()

@@ -370,16 +370,6 @@ int dense_fast_rf(int M, int N) {
   return best;
 }
 
-// Fewer than 64 tiles of 256 x 256: whether the split-K GEMM of the x.A path
-// is faster than 64-row tiles here. Measured over 16-1024 rows at [3840, 3840],
-// [3840, 10240] and [3584, 2560]: the split takes about 14 us + 0.95 us a
-// GFLOP, one round of 64-row tiles 5 us + 0.45 us a K stage (768 x 3840 x
-// 3840: 36 against 33 us; 256 rows: 22 against 30).
-bool dense_prefers_split(int M, int N, int K) {
-  const double split_us = 14.0 + 0.95 * (2e-9 * M * (double)N * K);
-  return split_us <= 5.0 + 0.45 * (K / DBK);
-}
-
 template <int RF>
 static void launch_rf(const QprojArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)(((a.M + 64 * RF - 1) / (64 * RF)) * ((a.N + DBN - 1) / DBN)));

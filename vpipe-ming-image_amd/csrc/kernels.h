@@ -118,6 +118,10 @@ hipError_t validate_attention_kernels();
 // row(c) = 16*grp[c/16] + c%16 (grp -1: a zero column). A is [R][K] bf16.
 // Up to this many projections share one x.A launch (q, k, v; w1, w3).
 constexpr int kMaxXaSources = 4;
+// A tile of the fast x.A kernel: 64*mr rows x 64*cj columns.
+struct XaTile {
+  int mr, cj;
+};
 struct LoraXaArgs {
   const uint16_t* x;
   long long ldx;
@@ -140,6 +144,10 @@ struct LoraXaArgs {
   // optional (fast kernel only): bias [n_cols] bf16, T = bf16(coef * sum +
   // bias) -- the dense split-K GEMM's ming_lin_bias
   const uint16_t* bias;
+  // fast kernel only: a dense weight's split-K GEMM. Column c is row c of
+  // A[0], coefficient 1 (grp and coef unused), in tiles of `tile`
+  bool ident;
+  XaTile tile;
 };
 hipError_t launch_lora_xa(const LoraXaArgs& a, hipStream_t s);
 
@@ -286,12 +294,18 @@ hipError_t launch_repack_fast(int bits, const uint32_t* codes,
 // x.A_live^T with split-K: `part` holds kslices * M * n_cols f32 (unused
 // when kslices == 1).
 int lora_xa_fast_slices(int M, int n_cols, int K);
-// The same kernel as a plain split-K bf16 GEMM y = x . W^T of a dense W
-// [N][K] (identity groups, coefficient 1): its slice count.
-int dense_xa_slices(int M, int N, int K);
 // Bytes of f32 partials launch_lora_xa_fast needs for kslices > 1 (whole
-// 256 x 128 tiles per slice, in the kernel's accumulator order); 0 otherwise.
+// tiles per slice, in the kernel's accumulator order); 0 otherwise.
 size_t lora_xa_part_bytes(int M, int n_cols, int kslices);
+size_t lora_xa_part_bytes(int M, int n_cols, int kslices, XaTile t);
+// The same kernel as a plain split-K bf16 GEMM y = x . W^T of a dense W
+// [N][K] of few tiles: its tile and slices, 0 slices where dense_fast.hip's
+// kernel is the faster one.
+struct DensePlan {
+  XaTile tile;
+  int slices;
+};
+DensePlan dense_split_plan(int M, int N, int K);
 hipError_t launch_lora_xa_fast(const LoraXaArgs& a, float* part, int kslices,
                                hipStream_t s);
 hipError_t launch_bf16_to_f16(const uint16_t* x, long long ldx, uint16_t* y,
@@ -303,10 +317,8 @@ hipError_t launch_bf16_to_f16(const uint16_t* x, long long ldx, uint16_t* y,
 // a.bias or a.g (fused SwiGLU) as QprojArgs says. N % 8 == 0, K % 64 == 0; x,
 // W, T and every B stack within 2 GiB of their base. rf: 64*rf rows a tile.
 hipError_t launch_dense_fast(const QprojArgs& a, int rf, hipStream_t s);
-// The tile height (rf) for a shape, and whether a dense projection of few
-// tiles is better split along K (launch_lora_xa_fast, identity groups).
+// The tile height (rf) for a shape.
 int dense_fast_rf(int M, int N);
-bool dense_prefers_split(int M, int N, int K);
 hipError_t validate_dense_fast_kernels();
 
 hipError_t validate_qproj_kernels();

@@ -765,10 +765,14 @@ __global__ void qproj_split_reduce_kernel(const QprojArgs a) {
 // stage t - 1 left and wait until stage t + 1 has landed; the MFMA waves
 // have then finished every read of stage t (steps 0-2 read it; step 3,
 // after the barrier, reads stage t + 1's first fragments).
+template <int MR, int CJ>
 __global__ __launch_bounds__(512, 1) void lora_xa_fast_kernel(const LoraXaArgs a, float* part,
                                                               int kslices) {
-  constexpr int STG = 256 * 8 + 128 * 8;         // x tile + A tile, 16-B chunks
-  constexpr int PER = 12;                        // 8 x + 4 A DMAs per DMA wave
+  constexpr int XR = 64 * MR, XC = 64 * CJ;      // rows and ranks of the tile
+  constexpr int XCH = XR * 8;                    // 16-B chunks of the x tile
+  constexpr int STG = XCH + XC * 8;              // x tile + A tile
+  constexpr int XD = 2 * MR, AD = 2 * CJ;        // DMAs per DMA wave per stage
+  constexpr int PER = XD + AD;
   __shared__ uint4 st0[STG], st1[STG], st2[STG];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -778,14 +782,14 @@ __global__ __launch_bounds__(512, 1) void lora_xa_fast_kernel(const LoraXaArgs a
   const int wm = rw & 1, wc = rw >> 1;
   int m0, c0, ks;
   {
-    const int tiles_m = (a.M + 255) / 256, tiles_c = (a.n_cols + 127) / 128;
+    const int tiles_m = (a.M + XR - 1) / XR, tiles_c = (a.n_cols + XC - 1) / XC;
     const int nb = (int)gridDim.x;
     const int q = nb / 8, rem = nb % 8;
     const int xcd = (int)blockIdx.x % 8, local = (int)blockIdx.x / 8;
     const int v = xcd * q + (xcd < rem ? xcd : rem) + local;
     const int tc = v % tiles_c, rest = v / tiles_c;
-    m0 = (rest % tiles_m) * 256;
-    c0 = tc * 128;
+    m0 = (rest % tiles_m) * XR;
+    c0 = tc * XC;
     ks = rest / tiles_m;
   }
   const int KT = a.K / 64;
@@ -795,47 +799,53 @@ __global__ __launch_bounds__(512, 1) void lora_xa_fast_kernel(const LoraXaArgs a
   const int mlast = a.M - 1;
 
   if (dma_wave) {
-    uint32_t xoff[8];
+    uint32_t xoff[XD];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int p = 64 * (8 * rw + i) + lane;
+    for (int i = 0; i < XD; ++i) {
+      const int p = 64 * (XD * rw + i) + lane;
       const int row = p >> 3;
       const int c = (p & 7) ^ ((row >> 1) & 7);
       int m = m0 + row;
       m = m < mlast ? m : mlast;
       xoff[i] = (uint32_t)(((long long)m * a.ldx + 8 * c) * 2);
     }
-    const int g_safe = a.grp[0];
-    uint32_t aoff[4];
-    int asrc[4];
+    const int g_safe = a.ident ? 0 : a.grp[0];
+    uint32_t aoff[AD];
+    int asrc[AD];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int p = 64 * (4 * rw + i) + lane;
+    for (int i = 0; i < AD; ++i) {
+      const int p = 64 * (AD * rw + i) + lane;
       const int r = p >> 3;
       const int c = (p & 7) ^ ((r >> 1) & 7);
       const int col = c0 + r;
-      const int g = col < a.n_cols ? a.grp[col >> 3] : -1;
-      const int gs = g < 0 ? g_safe : g;
-      const int row = 8 * (gs & 4095) + (g < 0 ? 0 : (col & 7));
+      int g, row;                                // stack (>> 12) and row of the column
+      if (a.ident) {
+        g = 0;
+        row = col < a.n_cols ? col : a.n_cols - 1;
+      } else {
+        const int gc = col < a.n_cols ? a.grp[col >> 3] : -1;
+        g = gc < 0 ? g_safe : gc;
+        row = 8 * (g & 4095) + (gc < 0 ? 0 : (col & 7));
+      }
       aoff[i] = (uint32_t)(((long long)row * a.K + 8 * c) * 2);
-      asrc[i] = __builtin_amdgcn_readfirstlane(gs >> 12);
+      asrc[i] = __builtin_amdgcn_readfirstlane(g >> 12);
     }
     auto issue = [&](int kt, const uint4* S) {
       const void* base = a.x + (long long)kt * 64;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) dma16_sb(base, xoff[i], lds_addr(S + 64 * (8 * rw + i)));
+      for (int i = 0; i < XD; ++i) dma16_sb(base, xoff[i], lds_addr(S + 64 * (XD * rw + i)));
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < AD; ++i)
         dma16_sb(a.A[asrc[i]] + (long long)kt * 64, aoff[i],
-                 lds_addr(S + 2048 + 64 * (4 * rw + i)));
+                 lds_addr(S + XCH + 64 * (AD * rw + i)));
     };
     // The fp16 copy of x (a.xh): the column blocks of one row tile and K
-    // slice split its 256 rows, so each element is converted once. Stage t
+    // slice split its rows, so each element is converted once. Stage t
     // is converted while it is in LDS (landed at the previous wait, its
     // buffer rewritten only after the next barrier): lane q takes chunk
     // q & 7 of rows r0 + q / 8 + 32 j.
-    const int tiles_c = (a.n_cols + 127) / 128, tc = c0 / 128;
-    const int r0 = 256 * tc / tiles_c, r1 = 256 * (tc + 1) / tiles_c;
+    const int tiles_c = (a.n_cols + XC - 1) / XC, tc = c0 / XC;
+    const int r0 = XR * tc / tiles_c, r1 = XR * (tc + 1) / tiles_c;
     const int q = 64 * rw + lane, qc = q & 7;
     uint32_t seen = 0;
     auto convert = [&](int t, const uint4* S) {
@@ -882,40 +892,40 @@ __global__ __launch_bounds__(512, 1) void lora_xa_fast_kernel(const LoraXaArgs a
     return;
   }
 
-  floatx16_t acc[4][2];
+  floatx16_t acc[MR][CJ];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MR; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < CJ; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
-  const bool live = c0 + 64 * wc < a.n_cols;
-  uint4 xb[4], ab[2];
-  auto read_frags = [&](const uint4* S, int kk, uint4 (&xv)[4], uint4 (&av)[2]) {
+  const bool live = c0 + 32 * CJ * wc < a.n_cols;
+  uint4 xb[MR], ab[CJ];
+  auto read_frags = [&](const uint4* S, int kk, uint4 (&xv)[MR], uint4 (&av)[CJ]) {
     const int c = 2 * kk + fk;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) xv[i] = S[swz8(128 * wm + 32 * i + fr, c)];
+    for (int i = 0; i < MR; ++i) xv[i] = S[swz8(32 * MR * wm + 32 * i + fr, c)];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) av[j] = S[2048 + swz8(64 * wc + 32 * j + fr, c)];
+    for (int j = 0; j < CJ; ++j) av[j] = S[XCH + swz8(32 * CJ * wc + 32 * j + fr, c)];
   };
   auto body = [&](const uint4* C, const uint4* Nx) {
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
-      uint4 xn[4], an[2];
+      uint4 xn[MR], an[CJ];
       if (kk < 3) read_frags(C, kk + 1, xn, an);
       else read_frags(Nx, 0, xn, an);
       if (live) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MR; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
+          for (int j = 0; j < CJ; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                 __builtin_bit_cast(bf16x8_t, ab[j]), __builtin_bit_cast(bf16x8_t, xb[i]),
                 acc[i][j], 0, 0, 0);
       }
 #pragma unroll
-      for (int g = 0; g < 6; ++g) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // DS read
+      for (int g = 0; g < (MR + CJ < MR * CJ ? MR + CJ : MR * CJ); ++g) {
+        __builtin_amdgcn_sched_group_barrier(0x100, MR + CJ <= MR * CJ ? 1 : 2, 0);   // DS read
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -924,9 +934,9 @@ __global__ __launch_bounds__(512, 1) void lora_xa_fast_kernel(const LoraXaArgs a
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) xb[i] = xn[i];
+      for (int i = 0; i < MR; ++i) xb[i] = xn[i];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) ab[j] = an[j];
+      for (int j = 0; j < CJ; ++j) ab[j] = an[j];
     }
   };
   ring_wait<0>();                                // stage 0 landed (the DMA waves' wait)
@@ -943,36 +953,37 @@ __global__ __launch_bounds__(512, 1) void lora_xa_fast_kernel(const LoraXaArgs a
   if (!live) return;
   if (kslices > 1) {
     // The partials in the accumulators' own order: slice ks, tile (row tile,
-    // column block), MFMA wave, fragment f = 8i + 4j + q, lane -- each store
+    // column block), MFMA wave, fragment f = (CJ i + j) 4 + q, lane -- each store
     // instruction writes 64 lanes x 16 B contiguous (the row-major layout
     // scattered every instruction over 32 rows). lora_xa_reduce_kernel reads
     // the same order.
-    const int tiles_c = (a.n_cols + 127) / 128;
-    const long long tile = (long long)(m0 / 256) * tiles_c + c0 / 128;
-    const long long ntiles = (long long)((a.M + 255) / 256) * tiles_c;
-    float4* pw = reinterpret_cast<float4*>(part) + (((ks * ntiles + tile) * 4 + rw) * 32) * 64 + lane;
+    const int tiles_c = (a.n_cols + XC - 1) / XC;
+    const long long tile = (long long)(m0 / XR) * tiles_c + c0 / XC;
+    const long long ntiles = (long long)((a.M + XR - 1) / XR) * tiles_c;
+    float4* pw = reinterpret_cast<float4*>(part) +
+                 (((ks * ntiles + tile) * 4 + rw) * (4 * MR * CJ)) * 64 + lane;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MR; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < CJ; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          pw[(8 * i + 4 * j + q) * 64] =
+          pw[(4 * (CJ * i + j) + q) * 64] =
               make_float4(acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
                           acc[i][j][4 * q + 3]);
     return;
   }
   // D[c][m]: lane owns row m, four consecutive ranks per register quad.
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + 128 * wm + 32 * i + fr;
+  for (int i = 0; i < MR; ++i) {
+    const int m = m0 + 32 * MR * wm + 32 * i + fr;
     if (m >= a.M) continue;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < CJ; ++j) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int c = c0 + 64 * wc + 32 * j + 8 * q + 4 * fk;
-        const float f = a.coef[c >> 3];
+        const int c = c0 + 32 * CJ * wc + 32 * j + 8 * q + 4 * fk;
+        const float f = a.ident ? 1.0f : a.coef[c >> 3];
         uint2 v;
         if (f == 0.0f) {
           v = make_uint2(0, 0);
@@ -1001,24 +1012,26 @@ __global__ __launch_bounds__(512, 1) void lora_xa_fast_kernel(const LoraXaArgs a
 // coalesced), one 16-byte store of T. Positions of row tiles past M or
 // column blocks past n_cols are skipped. 32-bit indices (the host keeps a
 // slice's float4 count below 2^31).
+template <int MR, int CJ>
 __global__ void lora_xa_reduce_kernel(const float* part, int kslices, int M,
                                       int n_cols, const LoraXaArgs a) {
-  const unsigned tiles_c = ((unsigned)n_cols + 127) / 128;
-  const unsigned ntiles = (((unsigned)M + 255) / 256) * tiles_c;
-  const unsigned total = ntiles * 8192u;             // float4s per slice
+  constexpr unsigned XR = 64 * MR, XC = 64 * CJ, FR = 4 * MR * CJ;
+  const unsigned tiles_c = ((unsigned)n_cols + XC - 1) / XC;
+  const unsigned ntiles = (((unsigned)M + XR - 1) / XR) * tiles_c;
+  const unsigned total = ntiles * (256u * FR);       // float4s per slice
   const bool st16 = (reinterpret_cast<uintptr_t>(a.t) & 15) == 0 && (a.ldt & 7) == 0;
   const float4* p4 = reinterpret_cast<const float4*>(part);
   for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < total / 2;
        t += gridDim.x * blockDim.x) {
-    // the float4 of accumulator lane fr: ((tile * 4 + wave) * 32 + f) * 64 + fr,
-    // f = 8 fi + 4 fj + fq; lane fr + 32 is 32 float4s on
+    // the float4 of accumulator lane fr: ((tile * 4 + wave) * FR + f) * 64 + fr,
+    // f = (CJ fi + fj) 4 + fq; lane fr + 32 is 32 float4s on
     const unsigned fr = t & 31, g = t >> 5;
     const unsigned i = g * 64 + fr;
-    const unsigned f = g & 31, wave = (g >> 5) & 3, tile = g >> 7;
-    const unsigned fi = f >> 3, fj = (f >> 2) & 1, fq = f & 3;
+    const unsigned f = g % FR, wave = (g / FR) & 3, tile = g / (4 * FR);
+    const unsigned fi = f / (4 * CJ), fj = (f >> 2) % CJ, fq = f & 3;
     const unsigned tm = tile / tiles_c, tc = tile - tm * tiles_c;
-    const unsigned m = 256 * tm + 128 * (wave & 1) + 32 * fi + fr;
-    const unsigned c = 128 * tc + 64 * (wave >> 1) + 32 * fj + 8 * fq;
+    const unsigned m = XR * tm + 32 * MR * (wave & 1) + 32 * fi + fr;
+    const unsigned c = XC * tc + 32 * CJ * (wave >> 1) + 32 * fj + 8 * fq;
     if (m >= (unsigned)M || c >= (unsigned)n_cols) continue;
     float4 s0 = p4[i], s1 = p4[i + 32];
     for (int k = 1; k < kslices; ++k) {
@@ -1027,7 +1040,7 @@ __global__ void lora_xa_reduce_kernel(const float* part, int kslices, int M,
       s0.x += v0.x; s0.y += v0.y; s0.z += v0.z; s0.w += v0.w;
       s1.x += v1.x; s1.y += v1.y; s1.z += v1.z; s1.w += v1.w;
     }
-    const float co = a.coef[c >> 3];
+    const float co = a.ident ? 1.0f : a.coef[c >> 3];
     uint4 o = make_uint4(0, 0, 0, 0);
     if (co != 0.0f && a.bias) {
       // the dense split-K GEMM with a bias (coef 1): one rounding
@@ -1358,38 +1371,109 @@ int lora_xa_fast_slices(int M, int n_cols, int K) {
   return ks < 1 ? 1 : ks;
 }
 
-// A dense projection through the x.A kernel: as many slices as fill about
-// one round of the chip, at least 8 K steps each.
-int dense_xa_slices(int M, int N, int K) {
-  const int tiles = ((M + 255) / 256) * ((N + 127) / 128);
-  const int KT = K / 64;
-  int ks = 256 / (tiles > 0 ? tiles : 1);
-  const int kmax = KT / 8 > 1 ? KT / 8 : 1;
-  if (ks > kmax) ks = kmax;
-  return ks < 1 ? 1 : ks;
+// The tile of an adapters' x.A over its fixed slices (same bits in each): the
+// 256 x 128 one stages the fewest bytes and is taken where its blocks fill
+// half the chip; a narrow stack or a short x leaves it on a few CUs (one
+// adapter of rank 16 at 4352 rows: 51 blocks, 42.3 us with its reduce) where
+// 64-row tiles spread out (19.9). Measured at 16-512 ranks, 100-16640 rows:
+// 512 ranks at 1493 rows (168 blocks) 23.5 against 25.5, at 1024 (112) 24.1
+// against 21.8.
+static XaTile xa_tile(int M, int n_cols, int kslices) {
+  const long long blocks = (long long)((M + 255) / 256) * ((n_cols + 127) / 128) * kslices;
+  if (blocks >= 136) return {4, 2};
+  return n_cols <= 64 ? XaTile{1, 1} : XaTile{1, 2};
 }
 
-size_t lora_xa_part_bytes(int M, int n_cols, int kslices) {
+size_t lora_xa_part_bytes(int M, int n_cols, int kslices, XaTile t) {
   if (kslices <= 1) return 0;
-  return (size_t)kslices * (size_t)((M + 255) / 256) * (size_t)((n_cols + 127) / 128) *
-         (256 * 128 * 4);
+  const size_t xr = 64 * t.mr, xc = 64 * t.cj;
+  return (size_t)kslices * (((size_t)M + xr - 1) / xr) * (((size_t)n_cols + xc - 1) / xc) *
+         (xr * xc * 4);
+}
+size_t lora_xa_part_bytes(int M, int n_cols, int kslices) {
+  return lora_xa_part_bytes(M, n_cols, kslices, xa_tile(M, n_cols, kslices));
+}
+
+// A dense projection of fewer than 64 tiles of 256 x 256 through the x.A
+// kernel: its tile and slices by a time model, and whether that beats one
+// round of dense_fast.hip's 64-row tiles (about 5 us + 0.72 us a K stage). The
+// model, us: a start, the larger of the staged bytes at the tile's rate and
+// the stages of a block in its rounds, and for a split its reduce launch and
+// the f32 partials, written and read at 5 TB/s; within 10% of what it was
+// fitted to, 16-1024 rows at [2304..10240] x [2560..10240] with the weights
+// rotated through more than the 256 MB cache, as a forward meets them. 16 rows
+// of [3840, 3840]: 13.5 us (64 x 64 in 4 slices; 256 x 128 in 8: 19.2), 231 of
+// [3584, 2560]: 17.7 (128 x 64 in 2; 21.4), 1024 of [3840, 3840]: 42.2 (256 x
+// 128 in 2; 64-row tiles of dense_fast 48.5).
+DensePlan dense_split_plan(int M, int N, int K) {
+  const int KT = K / 64;
+  DensePlan best = {{4, 2}, 0};
+  double cost = 5.0 + 0.72 * KT;
+  // the partials stay within what 256 x 128 tiles in one round would take
+  const int tiles = ((M + 255) / 256) * ((N + 127) / 128);
+  int kold = 256 / (tiles > 0 ? tiles : 1);
+  const int kmax = KT / 8 > 1 ? KT / 8 : 1;
+  if (kold > kmax) kold = kmax;
+  const size_t room = lora_xa_part_bytes(M, N, kold, {4, 2});
+  const int cus = device_cus();
+  const struct {
+    XaTile t;
+    int per_cu;                       // blocks a CU holds (LDS)
+    double start_us, bytes_us, stage_us;
+  } cand[5] = {{{4, 2}, 1, 2.0, 14e6, 0.84},
+               {{2, 2}, 1, 3.0, 11.5e6, 0.65},
+               {{2, 1}, 2, 2.5, 10e6, 0.5},
+               {{1, 2}, 2, 5.0, 10e6, 0.5},
+               {{1, 1}, 3, 4.5, 10e6, 0.36}};
+  for (const auto& c : cand) {
+    const long long n = (long long)((M + 64 * c.t.mr - 1) / (64 * c.t.mr)) *
+                        ((N + 64 * c.t.cj - 1) / (64 * c.t.cj));
+    for (int ks = 1; ks == 1 || KT / ks >= 4; ++ks) {
+      if (lora_xa_part_bytes(M, N, ks, c.t) > room) break;
+      const double staged = (double)n * KT * (c.t.mr + c.t.cj) * 8192.0 / c.bytes_us;
+      const double waits = (double)((n * ks + c.per_cu * cus - 1) / (c.per_cu * cus)) *
+                           ((KT + ks - 1) / ks) * c.stage_us;
+      double us = c.start_us + (staged > waits ? staged : waits);
+      if (ks > 1) us += 2.5 + 8.0 * ks * (double)M * N / 5e6;
+      if (us < cost) {
+        cost = us;
+        best = {c.t, ks};
+      }
+    }
+  }
+  return best;
+}
+
+template <int MR, int CJ>
+static hipError_t launch_xa_tiles(const LoraXaArgs& a, float* part, int kslices, hipStream_t s) {
+  constexpr int XR = 64 * MR, XC = 64 * CJ;
+  const long long tiles = (long long)((a.M + XR - 1) / XR) * ((a.n_cols + XC - 1) / XC);
+  // the reduce's 32-bit indexing: one thread per two float4s of a slice
+  const long long work = tiles * 1024 * MR * CJ;
+  if (kslices > 1 && (a.n_cols % 8 != 0 || work >= (1ll << 31))) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((lora_xa_fast_kernel<MR, CJ>), dim3((unsigned)(tiles * kslices)), dim3(512),
+                     0, s, a, part, kslices);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || kslices == 1) return e;
+  long long blocks = (work / 2 + 255) / 256;
+  if (blocks > 4096) blocks = 4096;
+  hipLaunchKernelGGL((lora_xa_reduce_kernel<MR, CJ>), dim3((unsigned)blocks), dim3(256), 0, s,
+                     part, kslices, a.M, a.n_cols, a);
+  return hipGetLastError();
 }
 
 hipError_t launch_lora_xa_fast(const LoraXaArgs& a, float* part, int kslices,
                                hipStream_t s) {
   if (a.M <= 0 || a.n_cols <= 0) return hipSuccess;
-  // the reduce's 32-bit indexing: one thread per float4 of a slice
-  const long long work = (long long)((a.M + 255) / 256) * ((a.n_cols + 127) / 128) * 8192;
-  if (kslices > 1 && (a.n_cols % 8 != 0 || work >= (1ll << 31))) return hipErrorInvalidValue;
-  const unsigned nblk = (unsigned)(((a.M + 255) / 256) * ((a.n_cols + 127) / 128) * kslices);
-  hipLaunchKernelGGL(lora_xa_fast_kernel, dim3(nblk), dim3(512), 0, s, a, part, kslices);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || kslices == 1) return e;
-  long long blocks = (work / 2 + 255) / 256;
-  if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(lora_xa_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s,
-                     part, kslices, a.M, a.n_cols, a);
-  return hipGetLastError();
+  const XaTile t = a.ident ? a.tile : xa_tile(a.M, a.n_cols, kslices);
+  switch (10 * t.mr + t.cj) {
+    case 11: return launch_xa_tiles<1, 1>(a, part, kslices, s);
+    case 12: return launch_xa_tiles<1, 2>(a, part, kslices, s);
+    case 21: return launch_xa_tiles<2, 1>(a, part, kslices, s);
+    case 22: return launch_xa_tiles<2, 2>(a, part, kslices, s);
+    case 42: return launch_xa_tiles<4, 2>(a, part, kslices, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_repack_fast(int bits, const uint32_t* codes,
@@ -1442,8 +1526,16 @@ hipError_t validate_qproj_fast_kernels() {
                        reinterpret_cast<const void*>(&bf16_to_f16_kernel),
                        reinterpret_cast<const void*>(&qproj_pair_kernel<4, 8, 4>),
                        reinterpret_cast<const void*>(&qproj_pair_kernel<8, 8, 4>),
-                       reinterpret_cast<const void*>(&lora_xa_fast_kernel),
-                       reinterpret_cast<const void*>(&lora_xa_reduce_kernel)};
+                       reinterpret_cast<const void*>(&lora_xa_fast_kernel<1, 1>),
+                       reinterpret_cast<const void*>(&lora_xa_reduce_kernel<1, 1>),
+                       reinterpret_cast<const void*>(&lora_xa_fast_kernel<1, 2>),
+                       reinterpret_cast<const void*>(&lora_xa_reduce_kernel<1, 2>),
+                       reinterpret_cast<const void*>(&lora_xa_fast_kernel<2, 1>),
+                       reinterpret_cast<const void*>(&lora_xa_reduce_kernel<2, 1>),
+                       reinterpret_cast<const void*>(&lora_xa_fast_kernel<2, 2>),
+                       reinterpret_cast<const void*>(&lora_xa_reduce_kernel<2, 2>),
+                       reinterpret_cast<const void*>(&lora_xa_fast_kernel<4, 2>),
+                       reinterpret_cast<const void*>(&lora_xa_reduce_kernel<4, 2>)};
   for (const void* f : fns) {
     const hipError_t e = hipFuncGetAttributes(&fa, f);
     if (e != hipSuccess) return e;

@@ -1022,14 +1022,13 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
               (uint64_t)M * (uint64_t)K * 2 <= (1ull << 31);
     any_fast = any_fast || fast[i];
   }
-  // Per projection: the fast route's K split on few tiles; a dense weight with no live adapter on few
-  // 256 x 256 tiles (the caption embedder: 15; the final layer's 64
-  // columns: 16) runs as the x.A path's split-K bf16 GEMM (identity column
-  // groups, coefficient 1) where that is the faster one; it and the general
-  // route write a gated projection into a plane of its own first, since y may
-  // be the gate itself.
+  // Per projection: the fast route's K split on few tiles; a dense weight with
+  // no live adapter on few 256 x 256 tiles (the caption embedder: 15; the final
+  // layer's 64 columns: 16) runs as the x.A path's split-K bf16 GEMM where that
+  // is the faster one; it and the general route write a gated projection into a
+  // plane of its own first, since y may be the gate itself.
   int split_ks[ming::kMaxXaSources] = {};
-  int dense_ks[ming::kMaxXaSources] = {};
+  ming::DensePlan dense_plan[ming::kMaxXaSources] = {};
   // every other dense projection: the dense route's tile height, 0 where its
   // 32-bit offsets or its 8-column stores do not fit (the general kernel)
   int dense_rf[ming::kMaxXaSources] = {};
@@ -1045,11 +1044,11 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
     const bool dense = q->bits == 16 && c->route != MING_ROUTE_GENERAL &&
                        (uint64_t)M * (uint64_t)ldx * 2 <= (1ull << 31) &&
                        (uint64_t)q->N * (uint64_t)K * 2 <= (1ull << 31);
-    if (dense && live_segs[i] == 0 && tiles < 64 && q->N % 64 == 0 &&
-        q->N <= 8 * ming::kMaxGroups && K % 64 == 0 && o.ldy <= (1 << 30) &&
-        ming::dense_prefers_split(M, q->N, K)) {
-      dense_ks[i] = ming::dense_xa_slices(M, q->N, K);
-      part_bytes = std::max(part_bytes, ming::lora_xa_part_bytes(M, q->N, dense_ks[i]));
+    if (dense && live_segs[i] == 0 && tiles < 64 && q->N % 64 == 0 && o.ldy <= (1 << 30))
+      dense_plan[i] = ming::dense_split_plan(M, q->N, K);
+    if (dense_plan[i].slices > 0) {
+      part_bytes = std::max(part_bytes, ming::lora_xa_part_bytes(M, q->N, dense_plan[i].slices,
+                                                                 dense_plan[i].tile));
     } else if (dense && q->N % 8 == 0 && tail_fits[i]) {
       dense_rf[i] = ming::dense_fast_rf(M, q->N);
     }
@@ -1203,15 +1202,12 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
                               : (double)q->N * K * q->bits / 8 + 4.0 * q->N * (K / 64);
     const int bk = fast[i] ? (q->bits == 4 ? kBF4 : kBF8)
                            : (q->bits == 4 ? kBQ4 : (q->bits == 8 ? kBQ8 : kBDense));
-    if (dense_ks[i] > 0) {
+    if (dense_plan[i].slices > 0) {
       ming::LoraXaArgs da{};
       da.x = x; da.ldx = ldx; da.A[0] = q->w16; da.K = K; da.M = M;
       da.n_cols = q->N; da.t = a.y; da.ldt = (int)a.ldy; da.bias = o.bias;
-      for (int gi = 0; gi < q->N / 8; ++gi) {
-        da.grp[gi] = (int16_t)gi;
-        da.coef[gi] = 1.0f;
-      }
-      const int dks = dense_ks[i];
+      da.ident = true; da.tile = dense_plan[i].tile;
+      const int dks = dense_plan[i].slices;
       MING_HIP(profiled(c, bk, base_flops, 2.0 * M * K + wbytes + 2.0 * M * q->N,
                         [&] { return ming::launch_lora_xa_fast(da, part, dks, c->stream); }),
                "dense split-K launch");
