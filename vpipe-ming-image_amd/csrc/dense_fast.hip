@@ -30,8 +30,9 @@ namespace {
 constexpr int DBN = 256, DBK = 64, NW = 8;
 
 // EPI: 0 plain; 1 a.bias added before the output's one rounding; 2 gated by
-// a.g (the fused SwiGLU). One instance each: with all three in one the
-// 256-row tile's epilogue spilled registers.
+// a.g (the fused SwiGLU); 3 plain, a.nw projections over one x. One instance
+// each: with the first three in one the 256-row tile's epilogue spilled
+// registers.
 template <int RF, int EPI>
 __global__ __launch_bounds__(64 * NW, 1) void dense_fast_kernel(const QprojArgs a) {
   constexpr int BMT = 64 * RF;
@@ -61,7 +62,14 @@ __global__ __launch_bounds__(64 * NW, 1) void dense_fast_kernel(const QprojArgs 
   const int tiles_m = (a.M + BMT - 1) / BMT;
   const int tiles_n = (a.N + DBN - 1) / DBN;
   int tm, tn;
-  tile_of_block((int)blockIdx.x, tiles_m, tiles_n, &tm, &tn);
+  tile_of_block((int)blockIdx.x, tiles_m, EPI == 3 ? a.nw * tiles_n : tiles_n, &tm, &tn);
+  int wsel = 0;                            // the tile's projection
+  if constexpr (EPI == 3) {
+    wsel = tn / tiles_n;
+    tn -= wsel * tiles_n;
+  }
+  const uint16_t* const w16 = EPI == 3 && wsel > 0 ? a.more[wsel - 1].w16 : a.w16;
+  uint16_t* const yout = EPI == 3 && wsel > 0 ? a.more[wsel - 1].y : a.y;
   const int m0 = tm * BMT, n0 = tn * DBN;
   const int mlast = a.M - 1, nlast = a.N - 1;
   const int KT = a.K / DBK;
@@ -183,7 +191,7 @@ __global__ __launch_bounds__(64 * NW, 1) void dense_fast_kernel(const QprojArgs 
   walk(
       KT,
       [&](int t, const uint4* S) {
-        const void* base = a.w16 + (long long)(t < KT ? t : KT - 1) * DBK;
+        const void* base = w16 + (long long)(t < KT ? t : KT - 1) * DBK;
 #pragma unroll
         for (int i = 0; i < WD; ++i) dma16_sb(base, woff[i], lds_addr(S + 64 * (WD * wave + i)));
       },
@@ -198,9 +206,9 @@ __global__ __launch_bounds__(64 * NW, 1) void dense_fast_kernel(const QprojArgs 
   int sg = 0;
   for (int i = 1; i < a.nseg; ++i)
     if (n0 >= a.seg[i].n_begin) sg = i;
-  const int chunks = a.seg[sg].chunks;
+  const QprojSeg& s = EPI == 3 && wsel > 0 ? a.more[wsel - 1].seg : a.seg[sg];
+  const int chunks = s.chunks;
   if (chunks > 0) {
-    const QprojSeg& s = a.seg[sg];
     const int grp0 = s.grp0;
     // a padding group's T columns are exactly 0: any finite B will do, the
     // first live group's
@@ -280,7 +288,7 @@ __global__ __launch_bounds__(64 * NW, 1) void dense_fast_kernel(const QprojArgs 
   constexpr int RROWS = 32 * RF;
   uint4* const E = ring + (RROWS * 8) * wave;
   uint2* const E2 = reinterpret_cast<uint2*>(E);
-  const bool st16 = (a.ldy & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
+  const bool st16 = (a.ldy & 7) == 0 && (reinterpret_cast<uintptr_t>(yout) & 15) == 0;
   const int cl = lane & 7;
 #pragma unroll
   for (int h = 0; h < JF / 2; ++h) {
@@ -339,7 +347,7 @@ __global__ __launch_bounds__(64 * NW, 1) void dense_fast_kernel(const QprojArgs 
             vp[e] = pack_bf16x2_rne(silu_f(bf16_lo(gp[e])) * bf16_lo(vp[e]),
                                     silu_f(bf16_hi(gp[e])) * bf16_hi(vp[e]));
         }
-        uint16_t* yp = a.y + (long long)mr * a.ldy + n;
+        uint16_t* yp = yout + (long long)mr * a.ldy + n;
         if (st16) {
           *reinterpret_cast<uint4*>(yp) = v;
         } else {
@@ -356,24 +364,34 @@ __global__ __launch_bounds__(64 * NW, 1) void dense_fast_kernel(const QprojArgs 
 // Rounds of the chip, one block a CU, times a block's time: about 24 + 10 rf
 // us for 60 K stages (one round, measured at [1280, 3840] x [3840, 3840]: rf 2
 // 44, rf 3 54, rf 4 64 us), the same ratio at other K.
-int dense_fast_rf(int M, int N) {
+static double dense_us(int M, int N, int nw, int rf) {
+  const long long tiles =
+      (long long)((M + 64 * rf - 1) / (64 * rf)) * ((N + DBN - 1) / DBN) * nw;
+  return (double)((tiles + 255) / 256) * (24 + 10 * rf);
+}
+
+int dense_fast_rf(int M, int N, int nw) {
   int best = 4;
-  double cost = 0.0;
-  for (int rf = 4; rf >= 1; --rf) {
-    const long long tiles = (long long)((M + 64 * rf - 1) / (64 * rf)) * ((N + DBN - 1) / DBN);
-    const double c = (double)((tiles + 255) / 256) * (24 + 10 * rf);
-    if (rf == 4 || c < cost) {
-      cost = c;
-      best = rf;
-    }
-  }
+  for (int rf = 3; rf >= 1; --rf)
+    if (dense_us(M, N, nw, rf) < dense_us(M, N, nw, best)) best = rf;
   return best;
+}
+
+// Fewer rounds of the chip in one launch than in one each: three of [2560,
+// 3840] x [3840, 3840] two of 256-row tiles for three of 192-row ones (a block
+// 1101 us with three launches, 1059 with one).
+bool dense_merge_pays(int M, int N, int nw) {
+  return dense_us(M, N, nw, dense_fast_rf(M, N, nw)) <
+         0.95 * nw * dense_us(M, N, 1, dense_fast_rf(M, N));
 }
 
 template <int RF>
 static void launch_rf(const QprojArgs& a, hipStream_t s) {
-  const dim3 grid((unsigned)(((a.M + 64 * RF - 1) / (64 * RF)) * ((a.N + DBN - 1) / DBN)));
-  if (a.bias)
+  const int nw = a.nw > 1 ? a.nw : 1;
+  const dim3 grid((unsigned)(((a.M + 64 * RF - 1) / (64 * RF)) * ((a.N + DBN - 1) / DBN) * nw));
+  if (nw > 1)
+    hipLaunchKernelGGL((dense_fast_kernel<RF, 3>), grid, dim3(64 * NW), 0, s, a);
+  else if (a.bias)
     hipLaunchKernelGGL((dense_fast_kernel<RF, 1>), grid, dim3(64 * NW), 0, s, a);
   else if (a.g)
     hipLaunchKernelGGL((dense_fast_kernel<RF, 2>), grid, dim3(64 * NW), 0, s, a);
@@ -383,7 +401,8 @@ static void launch_rf(const QprojArgs& a, hipStream_t s) {
 
 hipError_t launch_dense_fast(const QprojArgs& a, int rf, hipStream_t s) {
   if (a.M <= 0 || a.N <= 0) return hipSuccess;
-  if (a.N % 8 != 0 || a.K % 64 != 0 || a.kslices > 1 || a.yh || (a.bias && a.g))
+  if (a.N % 8 != 0 || a.K % 64 != 0 || a.kslices > 1 || a.yh || (a.bias && a.g) ||
+      (a.nw > 1 && (a.nw > 3 || a.nseg != 1 || a.bias || a.g)))
     return hipErrorInvalidValue;
   switch (rf) {
     case 1: launch_rf<1>(a, s); break;
@@ -400,7 +419,8 @@ static hipError_t validate_rf() {
   hipFuncAttributes fa;
   const void* fns[] = {reinterpret_cast<const void*>(&dense_fast_kernel<RF, 0>),
                        reinterpret_cast<const void*>(&dense_fast_kernel<RF, 1>),
-                       reinterpret_cast<const void*>(&dense_fast_kernel<RF, 2>)};
+                       reinterpret_cast<const void*>(&dense_fast_kernel<RF, 2>),
+                       reinterpret_cast<const void*>(&dense_fast_kernel<RF, 3>)};
   for (const void* f : fns) {
     const hipError_t e = hipFuncGetAttributes(&fa, f);
     if (e != hipSuccess) return e;

@@ -35,6 +35,16 @@ struct QprojSeg {
   const uint16_t* B;    // row (n - n_begin)
 };
 
+// A further projection of a merged launch: of the first one's shape, bits and
+// ldy, one segment, its groups in the first one's grp[].
+struct QprojMore {
+  const uint32_t* codes;
+  const uint32_t* sb;
+  const uint16_t* w16;
+  uint16_t* y;
+  QprojSeg seg;
+};
+
 struct QprojArgs {
   const uint16_t* x;
   long long ldx;
@@ -73,6 +83,10 @@ struct QprojArgs {
   const uint32_t* codes_u;
   const uint32_t* sb_u;
   QprojSeg seg_u;
+  // a merged launch (launch_qproj_merged): nw projections over one x, the
+  // second and third here; partials [nw][kslices][M][N]
+  int nw;
+  QprojMore more[2];
   // optional bias [N] bf16, added to the f32 result before the output's one
   // bf16 rounding (dense weights: ming_lin_bias)
   const uint16_t* bias;
@@ -278,6 +292,11 @@ hipError_t validate_gemv_kernels();
 // ---- the fast quantized route (qproj_fast.hip) --------------------------------
 // x is fp16 (carrying bf16 values), a.codes / a.sb the fast resident layout.
 hipError_t launch_qproj_fast(int bits, const QprojArgs& a, hipStream_t s);
+// Up to three projections over one x as one launch (the fields at QprojArgs::nw),
+// each one's bits those of its own: the same K slices, tiles by the rounds of
+// all. qproj_merge_pays: whether that is less time than one launch each.
+hipError_t launch_qproj_merged(int bits, const QprojArgs& a, hipStream_t s);
+bool qproj_merge_pays(int M, int N, int K, int nw);
 // K slices of a projection of few tiles, and its tile height (0: no split).
 int qproj_split_plan(int M, int N, int K, int* rf);
 // The gate and up projections of a SwiGLU in one launch (the fields after
@@ -316,9 +335,13 @@ hipError_t launch_bf16_to_f16(const uint16_t* x, long long ldx, uint16_t* y,
 // y = x . W^T (+ the LoRA tail), W = a.w16 [N][K] bf16, x bf16 at ldx, with
 // a.bias or a.g (fused SwiGLU) as QprojArgs says. N % 8 == 0, K % 64 == 0; x,
 // W, T and every B stack within 2 GiB of their base. rf: 64*rf rows a tile.
+// With a.nw > 1, that many projections over one x as one launch (no bias, no
+// gate), the others' w16, y and segment in a.more.
 hipError_t launch_dense_fast(const QprojArgs& a, int rf, hipStream_t s);
-// The tile height (rf) for a shape.
-int dense_fast_rf(int M, int N);
+// The tile height (rf) for nw projections of a shape, and whether one launch
+// for them is less time than one each.
+int dense_fast_rf(int M, int N, int nw = 1);
+bool dense_merge_pays(int M, int N, int nw);
 hipError_t validate_dense_fast_kernels();
 
 hipError_t validate_qproj_kernels();

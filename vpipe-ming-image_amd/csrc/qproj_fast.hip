@@ -101,8 +101,10 @@ __device__ __forceinline__ int wchunk(int n, int h) {
 // PAIR (launch_qproj_pair): the tile's 256 weight rows are 128 rows of the
 // gate weight (the first half of the waves) and the same 128 rows of the up
 // weight (the second half); the tail stages the gate's and the up projection's T chunks side by
-// side; the epilogue meets the two in LDS and writes only the SwiGLU.
-template <int BITS, bool SPLIT, bool PAIR, int RF, int NW>
+// side; the epilogue meets the two in LDS and writes only the SwiGLU. MULTI
+// (qproj_merged_kernel): a.nw projections over one x, their column tiles side
+// by side in the tile grid.
+template <int BITS, bool SPLIT, bool PAIR, int RF, int NW, bool MULTI = false>
 __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   constexpr int WCH = BITS == 4 ? 512 : 1024;    // 16-B code chunks per stage
   constexpr int CPR = BITS == 4 ? 2 : 4;         // code chunks per row
@@ -141,20 +143,28 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   const int tiles_n = (a.N + BNT - 1) / BNT;
   int tm, tn, blk = (int)blockIdx.x, ks = 0, kt0 = 0;
   int KT = a.K / BK;
+  const int tiles_all = MULTI ? a.nw * tiles_n : tiles_n;
   if constexpr (SPLIT) {
-    ks = blk / (tiles_m * tiles_n);
-    blk -= ks * (tiles_m * tiles_n);
+    ks = blk / (tiles_m * tiles_all);
+    blk -= ks * (tiles_m * tiles_all);
   }
-  tile_of_block(blk, tiles_m, tiles_n, &tm, &tn);
+  tile_of_block(blk, tiles_m, tiles_all, &tm, &tn);
+  int wsel = 0;                                  // MULTI: the tile's projection
+  if constexpr (MULTI) {
+    wsel = tn / tiles_n;
+    tn -= wsel * tiles_n;
+  }
   const int m0 = tm * BMT, n0 = tn * BNT;
   const int mlast = a.M - 1, nlast = a.N - 1;
   int sg = 0;                                    // the tile's segment
   for (int i = 1; i < a.nseg; ++i)
     if (n0 >= a.seg[i].n_begin) sg = i;
+  const QprojSeg& seg = MULTI && wsel > 0 ? a.more[wsel - 1].seg : a.seg[sg];
+  uint16_t* const yout = MULTI && wsel > 0 ? a.more[wsel - 1].y : a.y;
   if constexpr (SPLIT) {
     // the last slice also runs the LoRA tail, a chunk of it about 5/8 of a
     // stage: it takes that much less of K (at least one stage each)
-    const int total = KT + a.seg[sg].chunks * 5 / 8;
+    const int total = KT + seg.chunks * 5 / 8;
     auto bound = [&](int i) {
       const int b = total * i / a.kslices, m = KT - (a.kslices - i);
       return b < m ? b : m;
@@ -166,8 +176,12 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   // stage 0 of this block's K range
   const _Float16* __restrict__ x16 = reinterpret_cast<const _Float16*>(a.x) + (long long)kt0 * BK;
   const uint4* __restrict__ codes =
-      reinterpret_cast<const uint4*>(upw ? a.codes_u : a.codes) + (long long)kt0 * a.N * CPR;
-  const uint32_t* __restrict__ sbp = (upw ? a.sb_u : a.sb) + (long long)kt0 * a.N;
+      reinterpret_cast<const uint4*>(MULTI && wsel > 0 ? a.more[wsel - 1].codes
+                                     : upw           ? a.codes_u
+                                                     : a.codes) +
+      (long long)kt0 * a.N * CPR;
+  const uint32_t* __restrict__ sbp =
+      (MULTI && wsel > 0 ? a.more[wsel - 1].sb : upw ? a.sb_u : a.sb) + (long long)kt0 * a.N;
 
   // DMA sources for this lane, per stage (advance by k).
   // x tile: wave issues chunks q = 8*wave + i; lane p = 64q + lane.
@@ -388,12 +402,12 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   ring_wait<0>();                               // drained; LDS free
 
   // ---- LoRA tail: T and gathered B chunks of 32 ranks, same ring ----
-  const int chunks32 = (!SPLIT || ks == a.kslices - 1) ? a.seg[sg].chunks : 0;
+  const int chunks32 = (!SPLIT || ks == a.kslices - 1) ? seg.chunks : 0;
   if (chunks32 > 0) {
     // PAIR: the second half of the waves gathers the up projection's B (its segment, its
     // groups); both T chunks are staged for every wave
-    const QprojSeg& sw = upw ? a.seg_u : a.seg[sg];
-    const int t_col0 = a.seg[sg].t_col0;
+    const QprojSeg& sw = upw ? a.seg_u : seg;
+    const int t_col0 = seg.t_col0;
     const int ldb = sw.ldb;
     const int grp0 = sw.grp0;
     const int seg_nb = sw.n_begin, seg_ne = sw.n_end;
@@ -546,7 +560,8 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
         for (int q = 0; q < 4; ++q) {
           const int n = n0 + 32 * JT * wave + 32 * j + 8 * q + 4 * fk;
           if (n < a.N)
-            *reinterpret_cast<float4*>(a.part + ((long long)ks * a.M + m) * a.N + n) =
+            *reinterpret_cast<float4*>(
+                a.part + ((long long)(wsel * a.kslices + ks) * a.M + m) * a.N + n) =
                 make_float4(acc[j][i][4 * q + 0], acc[j][i][4 * q + 1], acc[j][i][4 * q + 2],
                             acc[j][i][4 * q + 3]);
         }
@@ -626,7 +641,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   // of one wave complete in order, so no barrier is needed inside.
   const int rg = wave * JT / 2;   // the 64-column region this wave writes and stores from
   uint4* const E = ring + 1024 * rg;
-  const bool st16 = (a.ldy & 7) == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
+  const bool st16 = (a.ldy & 7) == 0 && (reinterpret_cast<uintptr_t>(yout) & 15) == 0;
   const int cl = lane & 7;
   const int n = n0 + 64 * rg + 8 * cl;
   uint32_t seen = 0;   // magnitudes written to the fp16 copy (range_report)
@@ -679,7 +694,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
             vp[e] = pack_bf16x2_rne(silu_f(bf16_lo(gp[e])) * bf16_lo(vp[e]),
                                     silu_f(bf16_hi(gp[e])) * bf16_hi(vp[e]));
         }
-        uint16_t* yp = a.y + (long long)m * a.ldy + n;
+        uint16_t* yp = yout + (long long)m * a.ldy + n;
         if (st16) {
           *reinterpret_cast<uint4*>(yp) = v;
         } else {
@@ -712,19 +727,28 @@ __global__ __launch_bounds__(64 * NW, 1) void qproj_pair_kernel(const QprojArgs 
   qproj_fast_body<BITS, false, true, RF, NW>(a);
 }
 
-// The split projection's end: y = bf16(sum of the slices in order), then as
-// the epilogue: the fused SwiGLU bf16(silu(g) * y) and the fp16 copy.
+template <int BITS, bool SPLIT, int RF, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void qproj_merged_kernel(const QprojArgs a) {
+  qproj_fast_body<BITS, SPLIT, false, RF, NW, true>(a);
+}
+
+// The split projection's end (grid y: the projection of a merged launch): y =
+// bf16(sum of the slices in order), then as the epilogue: the fused SwiGLU
+// bf16(silu(g) * y) and the fp16 copy.
 // 32-bit indices: the host keeps M * N / 4 below 2^31.
 __global__ void qproj_split_reduce_kernel(const QprojArgs a) {
   const unsigned n4 = (unsigned)a.N >> 2;
   const unsigned total = (unsigned)a.M * n4;
   const size_t plane = (size_t)a.M * (size_t)a.N;
+  const unsigned w = blockIdx.y;
+  const float* const part = a.part + w * a.kslices * plane;
+  uint16_t* const y = w > 0 ? a.more[w - 1].y : a.y;
   uint32_t seen = 0;
   for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < total;
        i += gridDim.x * blockDim.x) {
     const unsigned m = i / n4;
     const unsigned n = (i - m * n4) * 4;
-    const float* p = a.part + (size_t)m * a.N + n;
+    const float* p = part + (size_t)m * a.N + n;
     float4 sum = *reinterpret_cast<const float4*>(p);
     for (int k = 1; k < a.kslices; ++k) {
       p += plane;
@@ -740,7 +764,7 @@ __global__ void qproj_split_reduce_kernel(const QprojArgs a) {
         vp[e] = pack_bf16x2_rne(silu_f(bf16_lo(gp[e])) * bf16_lo(vp[e]),
                                 silu_f(bf16_hi(gp[e])) * bf16_hi(vp[e]));
     }
-    *reinterpret_cast<uint2*>(a.y + (size_t)m * a.ldy + n) = make_uint2(vp[0], vp[1]);
+    *reinterpret_cast<uint2*>(y + (size_t)m * a.ldy + n) = make_uint2(vp[0], vp[1]);
     if (a.yh) {
       seen = range_track(range_track(seen, vp[0]), vp[1]);
       *reinterpret_cast<uint2*>(a.yh + (size_t)m * a.ldyh + n) =
@@ -1180,6 +1204,7 @@ constexpr TileCost kTiles[4] = {{8, 73.5}, {6, 56.0}, {4, 45.0}, {2, 35.5}};
 // in every tile height, so the bits do not depend on the plan.
 struct RowPlan {
   int rows_main, rf_rest;
+  double us;
 };
 
 // Least time in rounds of the chip, one tile a CU, over whole rounds of
@@ -1192,7 +1217,7 @@ static RowPlan plan_rows(int M, int tiles_n, int rf_min) {
   auto rounds = [&](long long rows_of_tiles) {
     return (double)((rows_of_tiles * tiles_n + cus - 1) / cus);
   };
-  RowPlan best = {M, 8};
+  RowPlan best = {M, 8, 0.0};
   double cost = rounds(tiles_m) * kTiles[0].us;
   const int all = (int)rounds(tiles_m);
   for (int k = 0; k < 4; ++k) {
@@ -1205,10 +1230,11 @@ static RowPlan plan_rows(int M, int tiles_n, int rf_min) {
       const double c = head + rounds((M - m1 * BM + 32 * t.rf - 1) / (32 * t.rf)) * t.us;
       if (c < cost) {
         cost = c;
-        best = {m1 * BM, t.rf};
+        best = {m1 * BM, t.rf, 0.0};
       }
     }
   }
+  best.us = cost;
   return best;
 }
 
@@ -1219,6 +1245,15 @@ static RowPlan plan_rows(int M, int tiles_n, int rf_min) {
 // tiles would take (one round, at least 6 stages each), so the partials stay
 // within what they would take. [256, 3840] x [3840, 3840]: rf 2 in 4 slices, 24.6
 // us, where rf 8 in 10 took 30.7; 16 rows 14.1 against 18.6. 0: no split.
+static constexpr TileCost kStages[3] = {{8, 0.96}, {4, 0.57}, {2, 0.45}};
+
+static double split_us(const TileCost& t, int M, int N, int K, int ks, int nw) {
+  const int cus = device_cus();
+  const int grid = ((M + 32 * t.rf - 1) / (32 * t.rf)) * ((N + BN - 1) / BN) * nw;
+  return (double)((grid * ks + cus - 1) / cus) * ((K / BK + ks - 1) / ks) * t.us +
+         1.6e-6 * (double)M * N * nw * ks;
+}
+
 int qproj_split_plan(int M, int N, int K, int* rf) {
   *rf = 8;
   const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
@@ -1227,23 +1262,31 @@ int qproj_split_plan(int M, int N, int K, int* rf) {
   int kmax = 256 / tiles;
   if (kmax > KT / 6) kmax = KT / 6;
   if (kmax < 2) return 0;
-  const int cus = device_cus();
-  const TileCost stage[3] = {{8, 0.96}, {4, 0.57}, {2, 0.45}};
   int best = 0;
   double cost = 0.0;
-  for (const TileCost& t : stage) {
-    const int grid = ((M + 32 * t.rf - 1) / (32 * t.rf)) * ((N + BN - 1) / BN);
+  for (const TileCost& t : kStages)
     for (int ks = 2; ks <= kmax; ++ks) {
-      const double c = (double)((grid * ks + cus - 1) / cus) * ((KT + ks - 1) / ks) * t.us +
-                       1.6e-6 * (double)M * N * ks;
+      const double c = split_us(t, M, N, K, ks, 1);
       if (best == 0 || c < cost) {
         cost = c;
         best = ks;
         *rf = t.rf;
       }
     }
-  }
   return best;
+}
+
+// One launch each against one for all. Split: the merged one fills its rounds
+// of blocks, and is two launches where there were two each (a w4 block at 203
+// rows 312 us with three, 288 with one). Unsplit: where the rounds of all are
+// fewer (three of [1280, 3840] x [3840, 3840]: 135 against 73.5 by the model; a
+// w8 block 577 us with three, 545 with one); equal rounds gain nothing (4352
+// rows measured 0.3% slower a forward when merged).
+bool qproj_merge_pays(int M, int N, int K, int nw) {
+  int rf = 0;
+  if (qproj_split_plan(M, N, K, &rf) > 0) return true;
+  const int tiles_n = (N + BN - 1) / BN;
+  return plan_rows(M, nw * tiles_n, 2).us < 0.95 * nw * plan_rows(M, tiles_n, 2).us;
 }
 
 template <int BITS, bool SPLIT, int RF, int NW>
@@ -1267,6 +1310,29 @@ static void launch_split(const QprojArgs& a, hipStream_t s) {
     case 2: launch_tiles<BITS, true, 2, 8>(a, s); break;
     case 4: launch_tiles<BITS, true, 4, 8>(a, s); break;
     default: launch_tiles<BITS, true, 8, 4>(a, s); break;
+  }
+}
+template <int BITS, bool SPLIT, int RF, int NW>
+static void launch_merged_tiles(const QprojArgs& a, hipStream_t s) {
+  const int tiles = ((a.M + 32 * RF - 1) / (32 * RF)) * ((a.N + BN - 1) / BN) * a.nw;
+  hipLaunchKernelGGL((qproj_merged_kernel<BITS, SPLIT, RF, NW>),
+                     dim3((unsigned)(SPLIT ? tiles * a.kslices : tiles)), dim3(64 * NW), 0, s, a);
+}
+template <int BITS>
+static void launch_merged_rows(const QprojArgs& a, int rf, hipStream_t s) {
+  switch (rf) {
+    case 2: launch_merged_tiles<BITS, false, 2, 8>(a, s); break;
+    case 4: launch_merged_tiles<BITS, false, 4, 8>(a, s); break;
+    case 6: launch_merged_tiles<BITS, false, 6, 8>(a, s); break;
+    default: launch_merged_tiles<BITS, false, 8, 4>(a, s); break;
+  }
+}
+template <int BITS>
+static void launch_merged_split(const QprojArgs& a, hipStream_t s) {
+  switch (a.split_rf) {
+    case 2: launch_merged_tiles<BITS, true, 2, 8>(a, s); break;
+    case 4: launch_merged_tiles<BITS, true, 4, 8>(a, s); break;
+    default: launch_merged_tiles<BITS, true, 8, 4>(a, s); break;
   }
 }
 template <int BITS, int RF, int NW>
@@ -1303,6 +1369,7 @@ static hipError_t launch_plan(const QprojArgs& a, const RowPlan& p, F&& rows) {
   if (a.g) h.g = a.g + r * a.ldg;
   if (a.yh) h.yh = a.yh + r * a.ldyh;
   if (a.t) h.t = a.t + r * a.ldt;
+  for (int i = 0; i + 1 < a.nw; ++i) h.more[i].y = a.more[i].y + r * a.ldy;
   rows(h, p.rf_rest);
   return hipGetLastError();
 }
@@ -1331,6 +1398,44 @@ hipError_t launch_qproj_fast(int bits, const QprojArgs& a, hipStream_t s) {
     else
       launch_rows<8>(m, rf, s);
   });
+}
+
+hipError_t launch_qproj_merged(int bits, const QprojArgs& a, hipStream_t s) {
+  if (a.M <= 0 || a.N <= 0) return hipSuccess;
+  if ((bits != 4 && bits != 8) || a.nw < 2 || a.nw > 3 || a.nseg != 1 || a.g || a.yh)
+    return hipErrorInvalidValue;
+  if (a.kslices > 1) {
+    if (!a.part || a.N % 4 != 0 || (long long)a.M * (a.N / 4) >= (1ll << 31) ||
+        a.K / BK < a.kslices)
+      return hipErrorInvalidValue;
+    QprojArgs m = a;
+    double cost = 0.0;
+    for (const TileCost& t : kStages) {
+      const double c = split_us(t, a.M, a.N, a.K, a.kslices, a.nw);
+      if (cost == 0.0 || c < cost) {
+        cost = c;
+        m.split_rf = t.rf;
+      }
+    }
+    if (bits == 4)
+      launch_merged_split<4>(m, s);
+    else
+      launch_merged_split<8>(m, s);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    long long blocks = ((long long)a.M * (a.N / 4) + 255) / 256;
+    if (blocks > 4096) blocks = 4096;
+    hipLaunchKernelGGL(qproj_split_reduce_kernel, dim3((unsigned)blocks, (unsigned)a.nw), dim3(256),
+                       0, s, a);
+    return hipGetLastError();
+  }
+  return launch_plan(a, plan_rows(a.M, a.nw * ((a.N + BN - 1) / BN), 2),
+                     [&](const QprojArgs& m, int rf) {
+                       if (bits == 4)
+                         launch_merged_rows<4>(m, rf, s);
+                       else
+                         launch_merged_rows<8>(m, rf, s);
+                     });
 }
 
 hipError_t launch_qproj_pair(int bits, const QprojArgs& a, hipStream_t s) {
@@ -1509,6 +1614,20 @@ hipError_t validate_qproj_fast_kernels() {
                        reinterpret_cast<const void*>(&qproj_fast_kernel<4, true, 2, 8>),
                        reinterpret_cast<const void*>(&qproj_fast_kernel<4, true, 4, 8>),
                        reinterpret_cast<const void*>(&qproj_fast_kernel<4, true, 8, 4>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<4, false, 2, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<4, false, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<4, false, 6, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<4, false, 8, 4>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<4, true, 2, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<4, true, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<4, true, 8, 4>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<8, false, 2, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<8, false, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<8, false, 6, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<8, false, 8, 4>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<8, true, 2, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<8, true, 4, 8>),
+                       reinterpret_cast<const void*>(&qproj_merged_kernel<8, true, 8, 4>),
                        reinterpret_cast<const void*>(&qproj_pair_kernel<4, 4, 8>),
                        reinterpret_cast<const void*>(&qproj_pair_kernel<4, 6, 8>),
                        reinterpret_cast<const void*>(&qproj_fast_kernel<8, false, 2, 8>),

@@ -1069,6 +1069,30 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
                     qs[0]->segs.size() == 1 && qs[1]->segs.size() == 1 &&
                     qa[0].seg[0].chunks == qa[1].seg[0].chunks &&
                     qp_used[0] + qp_used[1] <= ming::kMaxGroups;
+  // Two or three ungated projections of one shape on the fast route, or on the
+  // dense one (q, k and v), run as one launch where that takes fewer rounds of
+  // the chip, each with the bits of its own launch.
+  bool merged = !pair && (n == 2 || n == 3);
+  int groups_used = 0;
+  for (int i = 0; i < n && merged; ++i) {
+    groups_used += qp_used[i];
+    merged = fast[i] == fast[0] && (fast[i] || dense_rf[i] > 0) && !outs[i].gate &&
+             !outs[i].yh && !outs[i].bias && qs[i]->segs.size() == 1 &&
+             qs[i]->bits == qs[0]->bits && qs[i]->N == qs[0]->N && outs[i].ldy == outs[0].ldy;
+  }
+  merged = merged && groups_used <= ming::kMaxGroups &&
+           (fast[0] ? ming::qproj_merge_pays(M, qs[0]->N, K, n)
+                    : ming::dense_merge_pays(M, qs[0]->N, n));
+  if (merged && split_ks[0] >= 2) {
+    // all projections' partials at once: a stream that is being captured, where
+    // the buffer cannot grow, keeps to what it holds
+    const size_t all = (size_t)n * split_ks[0] * M * qs[0]->N * 4;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (all > c->part_bytes)
+      MING_HIP(hipStreamIsCapturing(c->stream, &st), "capture status");
+    merged = st == hipStreamCaptureStatusNone;
+    if (merged) part_bytes = std::max(part_bytes, all);
+  }
   // The fast route reads x as fp16 carrying the same (bf16) values: one
   // conversion serves every projection here.
   const bool need_xh = any_fast && !xh_src;
@@ -1167,6 +1191,54 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
     }
     c->eng.elementwise += 1;
     c->eng.gemm_paired += 1;
+    return ok();
+  }
+  if (merged) {
+    const ming_qweight* q = qs[0];
+    ming::QprojArgs& a = qa[0];
+    a.x = fast[0] ? xh : x; a.ldx = fast[0] ? K : ldx;
+    a.codes = q->codes_f; a.sb = q->sbf; a.w16 = q->w16;
+    a.y = outs[0].y; a.ldy = outs[0].ldy; a.M = M; a.N = q->N; a.K = K;
+    a.t = T; a.ldt = t_cols > 0 ? t_cols : 0; a.nseg = 1;
+    a.range = range_word(c);
+    a.nw = n;
+    if (split_ks[0] >= 2) {
+      a.part = part;
+      a.kslices = split_ks[0];
+    }
+    double flops = 0.0;
+    int used = qp_used[0];
+    for (int i = 0; i < n; ++i) {
+      flops += 2.0 * M * (double)q->N * K + tail_flops[i];
+      if (i == 0) continue;
+      ming::QprojMore& w = a.more[i - 1];
+      w.codes = qs[i]->codes_f; w.sb = qs[i]->sbf; w.w16 = qs[i]->w16; w.y = outs[i].y;
+      w.seg = qa[i].seg[0];
+      w.seg.grp0 += used;
+      for (int gi = 0; gi < qp_used[i]; ++gi) a.grp[used + gi] = qa[i].grp[gi];
+      used += qp_used[i];
+    }
+    const double wbytes = n * (q->bits == 16 ? 2.0 * q->N * K
+                                             : (double)q->N * K * q->bits / 8 +
+                                                   4.0 * q->N * (K / 64));
+    MING_HIP(profiled(c, q->bits == 4 ? kBF4 : q->bits == 8 ? kBF8 : kBDense, flops,
+                      2.0 * M * K + wbytes + 2.0 * n * M * q->N,
+                      [&] {
+                        return fast[0] ? ming::launch_qproj_merged(q->bits, a, c->stream)
+                                       : ming::launch_dense_fast(
+                                             a, ming::dense_fast_rf(M, q->N, n), c->stream);
+                      }),
+             "qproj merged launch");
+    for (int i = 0; i < n; ++i) {
+      if (outs[i].took_fast) *outs[i].took_fast = fast[i];
+      if (fast[i]) c->eng.gemm_fast += 1;
+      if (a.kslices >= 2) c->eng.gemm_split += 1;
+      if (q->bits == 4) c->eng.gemm_q4 += 1;
+      else if (q->bits == 8) c->eng.gemm_q8 += 1;
+      else c->eng.gemm_dense += 1;
+      c->eng.lora_proj += live_segs[i];
+      c->eng.gemm_flops += 2ull * (uint64_t)M * (uint64_t)q->N * (uint64_t)K + lora_flops[i];
+    }
     return ok();
   }
   for (int i = 0; i < n; ++i) {
