@@ -42,6 +42,6 @@ def test_merged_qkv_bits(ctx, monkeypatch, bits, Hd, rows):
     ctx.residual_add(xd, ob, rows, Hd)
     ctx.synchronize()
     assert np.array_equal(got, from_dev(xd))
-    for k, q in gp.items():
+    for q in gp.values():
         if hasattr(q, "close"):
             q.close()

@@ -35,14 +35,17 @@ namespace {
 // residual / conversion kernel. Roundings to bf16 take v_cvt_pk_bf16_f32
 // (round to nearest even; the bit-twiddled rounding's bits for every
 // non-NaN value), two VALU per pair fewer than the bit arithmetic.
-template <int LPR, int CPL, int MODE>
-__global__ __launch_bounds__(256, 5) void rmsnorm_kernel(
+// FEW (the residual modes at few rows, LPR 64): a row a block, so that they
+// spread over the CUs, and the gains and gates loaded beside the row: with a
+// few waves per CU the time is the chain of loads, and registers are free.
+template <int LPR, int CPL, int MODE, bool FEW>
+__global__ __launch_bounds__(FEW ? 64 : 256, FEW ? 1 : 5) void rmsnorm_kernel(
     const uint16_t* x, long long ldx, const uint16_t* __restrict__ w,
     uint16_t* y, long long ldy, uint16_t* h, long long ldh,
     const float* __restrict__ tg, int rows, int D, float eps, int* range) {
   constexpr int RPW = 64 / LPR;  // rows per wave
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int row = (blockIdx.x * 4 + wave) * RPW + lane / LPR;
+  const int row = (blockIdx.x * (FEW ? 1 : 4) + wave) * RPW + lane / LPR;
   const int sub = lane % LPR;
   const int nch = D >> 3;
   const bool live = row < rows;
@@ -52,14 +55,20 @@ __global__ __launch_bounds__(256, 5) void rmsnorm_kernel(
   // of the residual modes is read after it, which keeps their registers
   // inside 5 waves per SIMD (4352 rows of 3840 then fit one round).
   uint4 v[CPL], hv[CPL], wv[CPL];
+  float4 tv[FEW && MODE == 2 ? CPL : 1][2];
   float ss = 0.0f;
 #pragma unroll
   for (int i = 0; i < CPL; ++i) {
     const int c = sub + LPR * i;
     if (live && c < nch) {
       v[i] = *reinterpret_cast<const uint4*>(xr + 8 * c);
-      if constexpr (MODE <= 1) wv[i] = *reinterpret_cast<const uint4*>(w + 8 * c);
-      else hv[i] = *reinterpret_cast<const uint4*>(h + (long long)row * ldh + 8 * c);
+      if constexpr (MODE <= 1 || FEW) wv[i] = *reinterpret_cast<const uint4*>(w + 8 * c);
+      if constexpr (MODE >= 2)
+        hv[i] = *reinterpret_cast<const uint4*>(h + (long long)row * ldh + 8 * c);
+      if constexpr (FEW && MODE == 2) {
+        tv[i][0] = *reinterpret_cast<const float4*>(tg + 8 * c);
+        tv[i][1] = *reinterpret_cast<const float4*>(tg + 8 * c + 4);
+      }
     }
   }
 #pragma unroll
@@ -84,7 +93,7 @@ __global__ __launch_bounds__(256, 5) void rmsnorm_kernel(
   for (int i = 0; i < CPL; ++i) {
     const int c = sub + LPR * i;
     if (c < nch) {
-      if constexpr (MODE >= 2) wv[i] = *reinterpret_cast<const uint4*>(w + 8 * c);
+      if constexpr (MODE >= 2 && !FEW) wv[i] = *reinterpret_cast<const uint4*>(w + 8 * c);
       const uint32_t* u = &v[i].x;
       const uint32_t* wu = &wv[i].x;
       uint4 o;
@@ -114,8 +123,9 @@ __global__ __launch_bounds__(256, 5) void rmsnorm_kernel(
       } else {
         float t[8];
         if (MODE == 2) {
-          const float4 t0 = *reinterpret_cast<const float4*>(tg + 8 * c);
-          const float4 t1 = *reinterpret_cast<const float4*>(tg + 8 * c + 4);
+          const float4 t0 = FEW ? tv[FEW ? i : 0][0] : *reinterpret_cast<const float4*>(tg + 8 * c);
+          const float4 t1 =
+              FEW ? tv[FEW ? i : 0][1] : *reinterpret_cast<const float4*>(tg + 8 * c + 4);
           t[0] = t0.x; t[1] = t0.y; t[2] = t0.z; t[3] = t0.w;
           t[4] = t1.x; t[5] = t1.y; t[6] = t1.z; t[7] = t1.w;
         }
@@ -145,8 +155,8 @@ __global__ __launch_bounds__(256, 5) void rmsnorm_kernel(
 // registers instead of being read back. Every expression and both
 // reductions are rmsnorm_kernel's at the same LPR / CPL, so the result is
 // bit-identical to the two launches it replaces.
-template <int LPR, int CPL, bool GATED>
-__global__ __launch_bounds__(256, 5) void norm_residual_norm_kernel(
+template <int LPR, int CPL, bool GATED, bool FEW>
+__global__ __launch_bounds__(FEW ? 64 : 256, FEW ? 1 : 5) void norm_residual_norm_kernel(
     const uint16_t* sub, long long lds, const uint16_t* __restrict__ wpost,
     uint16_t* h, long long ldh, const float* __restrict__ tg,
     const uint16_t* __restrict__ wpre, uint16_t* y, long long ldy, uint16_t* yh,
@@ -154,12 +164,14 @@ __global__ __launch_bounds__(256, 5) void norm_residual_norm_kernel(
   constexpr int RPW = 64 / LPR;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // rows wave-uniform at LPR 64
-  const int row = (blockIdx.x * 4 + wave) * RPW + lane / LPR;
+  const int row = (blockIdx.x * (FEW ? 1 : 4) + wave) * RPW + lane / LPR;
   const int sb = lane % LPR;
   const int nch = D >> 3;
   const bool live = row < rows;
   const long long rr = live ? row : 0;
   uint4 v[CPL], hv[CPL];
+  uint4 w1v[FEW ? CPL : 1], w2v[FEW ? CPL : 1];
+  float4 tv[FEW && GATED ? CPL : 1][2];
   float ss = 0.0f;
 #pragma unroll
   for (int i = 0; i < CPL; ++i) {
@@ -167,6 +179,14 @@ __global__ __launch_bounds__(256, 5) void norm_residual_norm_kernel(
     if (live && c < nch) {
       v[i] = *reinterpret_cast<const uint4*>(sub + rr * lds + 8 * c);
       hv[i] = *reinterpret_cast<const uint4*>(h + rr * ldh + 8 * c);
+      if constexpr (FEW) {
+        w1v[i] = *reinterpret_cast<const uint4*>(wpost + 8 * c);
+        w2v[i] = *reinterpret_cast<const uint4*>(wpre + 8 * c);
+        if constexpr (GATED) {
+          tv[i][0] = *reinterpret_cast<const float4*>(tg + 8 * c);
+          tv[i][1] = *reinterpret_cast<const float4*>(tg + 8 * c + 4);
+        }
+      }
     }
   }
 #pragma unroll
@@ -191,7 +211,7 @@ __global__ __launch_bounds__(256, 5) void norm_residual_norm_kernel(
   for (int i = 0; i < CPL; ++i) {
     const int c = sb + LPR * i;
     if (live && c < nch) {
-      const uint4 wv = *reinterpret_cast<const uint4*>(wpost + 8 * c);
+      const uint4 wv = FEW ? w1v[FEW ? i : 0] : *reinterpret_cast<const uint4*>(wpost + 8 * c);
       const uint32_t* u = &v[i].x;
       const uint32_t* wu = &wv.x;
       uint32_t ou[4];
@@ -203,8 +223,9 @@ __global__ __launch_bounds__(256, 5) void norm_residual_norm_kernel(
       }
       float t[8];
       if constexpr (GATED) {
-        const float4 t0 = *reinterpret_cast<const float4*>(tg + 8 * c);
-        const float4 t1 = *reinterpret_cast<const float4*>(tg + 8 * c + 4);
+        const float4 t0 = FEW ? tv[FEW ? i : 0][0] : *reinterpret_cast<const float4*>(tg + 8 * c);
+        const float4 t1 =
+            FEW ? tv[FEW ? i : 0][1] : *reinterpret_cast<const float4*>(tg + 8 * c + 4);
         t[0] = t0.x; t[1] = t0.y; t[2] = t0.z; t[3] = t0.w;
         t[4] = t1.x; t[5] = t1.y; t[6] = t1.z; t[7] = t1.w;
       }
@@ -238,7 +259,7 @@ __global__ __launch_bounds__(256, 5) void norm_residual_norm_kernel(
   for (int i = 0; i < CPL; ++i) {
     const int c = sb + LPR * i;
     if (c < nch) {
-      const uint4 wv = *reinterpret_cast<const uint4*>(wpre + 8 * c);
+      const uint4 wv = FEW ? w2v[FEW ? i : 0] : *reinterpret_cast<const uint4*>(wpre + 8 * c);
       const uint32_t* u = &hv[i].x;
       const uint32_t* wu = &wv.x;
       uint4 o;
@@ -488,6 +509,12 @@ __global__ __launch_bounds__(256) void llm_qk_norm_rope_kernel(
 
 }  // namespace
 
+// Where the residual kernels take a row a block (FEW): rows of 65 to 512
+// 16-byte chunks, while 8 waves a CU hold them all. A block's two launches at
+// width 3840, together: 203 rows 24 us, now 17; 512 27 and 18; 1280 32 and 25;
+// 2048 39 and 31; 3072 45 either way; 4352 60 against 64.
+static bool few_rows(int rows, int nch) { return rows <= 2048 && nch > 64 && nch <= 512; }
+
 hipError_t launch_rmsnorm_ex(int mode, const uint16_t* x, long long ldx, const uint16_t* w,
                              uint16_t* y, long long ldy, uint16_t* h, long long ldh,
                              const float* tg, int rows, int D, float eps,
@@ -495,12 +522,18 @@ hipError_t launch_rmsnorm_ex(int mode, const uint16_t* x, long long ldx, const u
   if (rows <= 0) return hipSuccess;
   const int nch = D / 8;
   if (D % 8 != 0 || nch > 64 * 16 || mode < 0 || mode > 3) return hipErrorInvalidValue;
-#define MING_RMS_M(LPR, CPL, MODE)                                                \
-  hipLaunchKernelGGL((rmsnorm_kernel<LPR, CPL, MODE>), dim3((rows + rpb - 1) / rpb), \
-                     dim3(256), 0, s, x, ldx, w, y, ldy, h, ldh, tg, rows, D, eps, range)
+  const bool few = mode >= 2 && few_rows(rows, nch);
+#define MING_RMS_L(LPR, CPL, MODE, FEW)                                                \
+  hipLaunchKernelGGL((rmsnorm_kernel<LPR, CPL, MODE, FEW>), dim3((rows + rpb - 1) / rpb), \
+                     dim3(FEW ? 64 : 256), 0, s, x, ldx, w, y, ldy, h, ldh, tg, rows, D, eps, range)
+#define MING_RMS_M(LPR, CPL, MODE)                                             \
+  do {                                                                         \
+    if (few) MING_RMS_L(LPR, CPL, MODE, (MODE >= 2 && ((CPL) == 4 || (CPL) == 8))); \
+    else MING_RMS_L(LPR, CPL, MODE, false);                                    \
+  } while (0)
 #define MING_RMS(LPR, CPL)                                                     \
   do {                                                                         \
-    const int rpb = 4 * (64 / (LPR));                                          \
+    const int rpb = few ? 1 : 4 * (64 / (LPR));                                \
     if (mode == 0) MING_RMS_M(LPR, CPL, 0);                                    \
     else if (mode == 1) MING_RMS_M(LPR, CPL, 1);                               \
     else if (mode == 2) MING_RMS_M(LPR, CPL, 2);                               \
@@ -515,6 +548,7 @@ hipError_t launch_rmsnorm_ex(int mode, const uint16_t* x, long long ldx, const u
   else MING_RMS(64, 16);
 #undef MING_RMS
 #undef MING_RMS_M
+#undef MING_RMS_L
   return hipGetLastError();
 }
 
@@ -526,13 +560,19 @@ hipError_t launch_norm_residual_norm(const uint16_t* sub, long long lds, const u
   if (rows <= 0) return hipSuccess;
   const int nch = D / 8;
   if (D % 8 != 0 || nch > 64 * 16) return hipErrorInvalidValue;
-#define MING_NRN_G(LPR, CPL, G)                                                          \
-  hipLaunchKernelGGL((norm_residual_norm_kernel<LPR, CPL, G>), dim3((rows + rpb - 1) / rpb), \
-                     dim3(256), 0, s, sub, lds, wpost, h, ldh, tg, wpre, y, ldy, yh, ldyh,   \
-                     rows, D, eps, range)
+  const bool few = few_rows(rows, nch);
+#define MING_NRN_L(LPR, CPL, G, FEW)                                                     \
+  hipLaunchKernelGGL((norm_residual_norm_kernel<LPR, CPL, G, FEW>),                      \
+                     dim3((rows + rpb - 1) / rpb), dim3(FEW ? 64 : 256), 0, s, sub, lds, \
+                     wpost, h, ldh, tg, wpre, y, ldy, yh, ldyh, rows, D, eps, range)
+#define MING_NRN_G(LPR, CPL, G)                                                \
+  do {                                                                         \
+    if (few) MING_NRN_L(LPR, CPL, G, ((CPL) == 4 || (CPL) == 8));              \
+    else MING_NRN_L(LPR, CPL, G, false);                                       \
+  } while (0)
 #define MING_NRN(LPR, CPL)                                                     \
   do {                                                                         \
-    const int rpb = 4 * (64 / (LPR));                                          \
+    const int rpb = few ? 1 : 4 * (64 / (LPR));                                \
     if (tg) MING_NRN_G(LPR, CPL, true);                                        \
     else MING_NRN_G(LPR, CPL, false);                                          \
   } while (0)
@@ -546,6 +586,7 @@ hipError_t launch_norm_residual_norm(const uint16_t* sub, long long lds, const u
   else MING_NRN(64, 16);
 #undef MING_NRN
 #undef MING_NRN_G
+#undef MING_NRN_L
   return hipGetLastError();
 }
 
@@ -626,19 +667,24 @@ namespace ming {
 hipError_t validate_norm_kernels() {
   hipFuncAttributes fa;
   const void* fns[] = {
-#define MING_RMS_ALL(LPR, CPL)                                      \
-  reinterpret_cast<const void*>(&rmsnorm_kernel<LPR, CPL, 0>),      \
-      reinterpret_cast<const void*>(&rmsnorm_kernel<LPR, CPL, 1>),  \
-      reinterpret_cast<const void*>(&rmsnorm_kernel<LPR, CPL, 2>),  \
-      reinterpret_cast<const void*>(&rmsnorm_kernel<LPR, CPL, 3>)
+#define MING_RMS_ALL(LPR, CPL)                                            \
+  reinterpret_cast<const void*>(&rmsnorm_kernel<LPR, CPL, 0, false>),     \
+      reinterpret_cast<const void*>(&rmsnorm_kernel<LPR, CPL, 1, false>), \
+      reinterpret_cast<const void*>(&rmsnorm_kernel<LPR, CPL, 2, false>), \
+      reinterpret_cast<const void*>(&rmsnorm_kernel<LPR, CPL, 3, false>)
       MING_RMS_ALL(8, 1),  MING_RMS_ALL(16, 1), MING_RMS_ALL(32, 1), MING_RMS_ALL(64, 1),
       MING_RMS_ALL(64, 4), MING_RMS_ALL(64, 8), MING_RMS_ALL(64, 16),
+      reinterpret_cast<const void*>(&rmsnorm_kernel<64, 4, 2, true>),
+      reinterpret_cast<const void*>(&rmsnorm_kernel<64, 4, 3, true>),
+      reinterpret_cast<const void*>(&rmsnorm_kernel<64, 8, 2, true>),
+      reinterpret_cast<const void*>(&rmsnorm_kernel<64, 8, 3, true>),
 #undef MING_RMS_ALL
-#define MING_NRN_ALL(LPR, CPL)                                                  \
-  reinterpret_cast<const void*>(&norm_residual_norm_kernel<LPR, CPL, true>),    \
-      reinterpret_cast<const void*>(&norm_residual_norm_kernel<LPR, CPL, false>)
-      MING_NRN_ALL(8, 1),  MING_NRN_ALL(16, 1), MING_NRN_ALL(32, 1), MING_NRN_ALL(64, 1),
-      MING_NRN_ALL(64, 4), MING_NRN_ALL(64, 8), MING_NRN_ALL(64, 16),
+#define MING_NRN_ALL(LPR, CPL, FEW)                                                  \
+  reinterpret_cast<const void*>(&norm_residual_norm_kernel<LPR, CPL, true, FEW>),    \
+      reinterpret_cast<const void*>(&norm_residual_norm_kernel<LPR, CPL, false, FEW>)
+      MING_NRN_ALL(8, 1, false),  MING_NRN_ALL(16, 1, false), MING_NRN_ALL(32, 1, false),
+      MING_NRN_ALL(64, 1, false), MING_NRN_ALL(64, 4, false), MING_NRN_ALL(64, 8, false),
+      MING_NRN_ALL(64, 16, false), MING_NRN_ALL(64, 4, true), MING_NRN_ALL(64, 8, true),
 #undef MING_NRN_ALL
       reinterpret_cast<const void*>(&rope_table_kernel),
       reinterpret_cast<const void*>(&qk_norm_rope_kernel),
