@@ -78,7 +78,7 @@ typedef struct ming_engagement {
 /* Kernel routes for quantized projections. AUTO takes the fast route
  * (fp16 activations, DMA-fed LDS ring, fragment dequant) whenever the
  * weight's scales and biases are exact in fp16, and a GEMV (each weight
- * streamed once, f32 dot products) for M <= 8 rows with no live adapter, as
+ * streamed once, f32 sums) for M <= 8 rows with no live adapter, as
  * the adaLN and timestep projections run at M = 1. GENERAL always takes the
  * general kernel. Both multiply fp16 activations: bf16 values are carried
  * exactly at magnitudes in [2^-17, 2^16); smaller ones are cut toward zero
