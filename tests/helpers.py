@@ -2,8 +2,11 @@
 device moves of bf16 bit patterns, and the projection problem builder."""
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 
+import ming_dit_amd as m
 import oracle as orc
 
 # BASELINE config 2's adapter set.
@@ -194,3 +197,14 @@ def build_model(ctx, seed, H=256, NH=2, F=512, n_layers=2, n_refiner=1,
         setattr(d, name, m._h(obj))
     model = m.Model(ctx, d, cb, mb, keep=keep + [dev, cb, mb])
     return mo, model
+
+
+# ---- the launch plans (kernels.h), by their exported C++ names ----
+class RowPlan(C.Structure):
+    _fields_ = [("rows_main", C.c_int), ("rf_rest", C.c_int), ("us", C.c_double)]
+
+
+def plan_rows(M, tiles_n, stages, pair):
+    f = m.lib()._ZN4ming9plan_rowsEiiib
+    f.argtypes, f.restype = [C.c_int, C.c_int, C.c_int, C.c_bool], RowPlan
+    return f(M, tiles_n, stages, pair)

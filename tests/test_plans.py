@@ -1,0 +1,34 @@
+"""The launch plans, which choose tile heights and K slices by size alone: on the
+CPU (without a device they count the MI355X's 256 CUs), through the library's
+own symbols."""
+import pytest
+
+from helpers import plan_rows
+
+SHAPES = [(M, tn, st) for M in (1, 63, 300, 700, 1280, 2085, 4352, 8320, 16640)
+          for tn in (1, 8, 15, 40, 60, 80, 129) for st in (1, 4, 16, 60, 165)]
+
+
+@pytest.mark.parametrize("pair", [False, True])
+def test_row_plans_cover_the_rows(pair):
+    for M, tn, st in SHAPES:
+        p = plan_rows(M, tn, st, pair)
+        assert p.rows_main == M or (p.rows_main % 256 == 0 and 0 <= p.rows_main < M), (M, tn, st)
+        assert p.rf_rest in ((8, 6, 4) if pair else (8, 6, 4, 2)), (M, tn, st)
+
+
+def test_row_plans_count_k():
+    """A short K leaves a second launch little to gain for its start: plans that
+    are two launches at K = 3840 are one at K = 64."""
+    two = [s for s in ((5600, 40), (8320, 40), (16640, 40)) if 0 < plan_rows(*s, 60, False).rows_main < s[0]]
+    assert two
+    for M, tn in two:
+        assert plan_rows(M, tn, 1, False).rows_main in (0, M)
+    # 4096 rows of [10240, 64]: one launch of a lower height (28.5 us, 36.2 as
+    # 256-row tiles and then 192)
+    assert plan_rows(4096, 40, 1, False).rows_main == 0
+    # 2560 rows of [10240, 3840]: one launch of 256-row tiles (171.8 us, 178.2)
+    assert plan_rows(2560, 40, 60, False).rows_main == 2560
+    # a paired launch's 4352 rows: five whole rounds, then 128-row tiles
+    p = plan_rows(4352, 80, 60, True)
+    assert (p.rows_main, p.rf_rest) == (4096, 4)

@@ -297,6 +297,16 @@ hipError_t launch_qproj_fast(int bits, const QprojArgs& a, hipStream_t s);
 // all. qproj_merge_pays: whether that is less time than one launch each.
 hipError_t launch_qproj_merged(int bits, const QprojArgs& a, hipStream_t s);
 bool qproj_merge_pays(int M, int N, int K, int nw);
+// The rows of an unsplit launch: the first rows_main as 256-row tiles, the others
+// as tiles of 32 * rf_rest, and the time that takes by the plan's model. Each
+// output element is computed by the same MFMA sequence in every tile height, so
+// the bits do not depend on the plan. tiles_n columns of tiles, stages of K (64)
+// and the LoRA tail; pair: the paired launch (256, 192 and 128 rows).
+struct RowPlan {
+  int rows_main, rf_rest;
+  double us;
+};
+RowPlan plan_rows(int M, int tiles_n, int stages, bool pair);
 // K slices of a projection of few tiles, and its tile height (0: no split).
 int qproj_split_plan(int M, int N, int K, int* rf);
 // The gate and up projections of a SwiGLU in one launch (the fields after

@@ -1194,56 +1194,90 @@ static int device_cus() {
   return cached[dev];
 }
 
-// Rows per tile. A tile of 32*rf rows over 60 K stages takes, in one round of
-// the chip, about 35.5, 45, 56 and 73.5 us at rf 2, 4, 6 and 8 (w4, [M, 3840] x
-// [3840, 3840], M = 300..1493; other K in proportion): rf 8 is the best rate
-// for a full chip (1.15x the MFMA time), the lower tiles fill it where 256
-// rows leave it idle (1280 rows: 75 tiles, 75.5 -> 49.8 us with 150 of rf 4).
-// rf 2 to 6 run eight waves, two a SIMD, each 32 columns: 49.8 against 53.2 us
-// with four waves at rf 4; at rf 8 their reads of x would fill the LDS.
+// Rows per tile. A launch of `tiles` tiles of 32*rf rows takes a start, a full
+// round's time for every whole round of the chip (one tile a CU), and for the
+// last one less while it leaves CUs idle: the others then clock higher and
+// share the memory with fewer. Per round a part of its own (prologue, epilogue,
+// store) and a part a K stage, us, fitted to 600 launches at K = 64 to 10240
+// and 60 to 1050 tiles, the paired launch's to 240; within 3% on the average
+// (rf 2, two blocks a CU, 5%). Of w4: w8 takes 1.03 to 1.06 of it at every
+// height. rf 8 is the best rate for a full chip, the lower tiles fill it where
+// 256 rows leave it idle (1280 rows of [3840, 3840]: 75 tiles, 75.5 -> 49.8 us
+// with 150 of rf 4). rf 2 to 6 run eight waves, two a SIMD, each 32 columns:
+// 49.8 against 53.2 us with four waves at rf 4; at rf 8 their reads of x would
+// fill the LDS.
 struct TileCost {
   int rf;
-  double us;
+  double full0, full, few0, few;   // a full round, one of at most half of the CUs
 };
-constexpr TileCost kTiles[4] = {{8, 73.5}, {6, 56.0}, {4, 45.0}, {2, 35.5}};
+constexpr TileCost kTiles[4] = {{8, 8.2, 1.510, 7.6, 1.027},
+                                {6, 5.7, 1.227, 4.1, 0.797},
+                                {4, 4.7, 0.867, 2.5, 0.602},
+                                {2, 2.3, 0.477, 1.3, 0.437}};
+constexpr TileCost kPairTiles[3] = {{8, 8.5, 1.380, 8.5, 0.930},
+                                    {6, 5.5, 1.110, 5.0, 0.680},
+                                    {4, 4.4, 0.770, 3.0, 0.530}};
 
-// The rows of a launch: the first rows_main as 256-row tiles, the others as
-// tiles of rf_rest. Each output element is computed by the same MFMA sequence
-// in every tile height, so the bits do not depend on the plan.
-struct RowPlan {
-  int rows_main, rf_rest;
-  double us;
-};
-
-// Least time in rounds of the chip, one tile a CU, over whole rounds of
-// 256-row tiles followed by one of the heights (a second launch costs about
-// 3 us). 4352 rows of a paired launch (80 column tiles): 16 tile rows in five
-// rounds, then 256 rows as rf 4 in one.
-static RowPlan plan_rows(int M, int tiles_n, int rf_min) {
+static double tiles_us(const TileCost& t, long long tiles, int stages) {
   const int cus = device_cus();
+  const double full = t.full0 + t.full * stages, few = t.few0 + t.few * stages;
+  const double fill = (double)(tiles % cus) / cus;
+  double us = 5.0 + (double)(tiles / cus) * full;
+  if (fill > 0.0) us += few + (fill > 0.5 ? (full - few) * (fill - 0.5) * 2.0 : 0.0);
+  return us;
+}
+
+// One launch of one height, or the 256-row tile rows that fill some whole
+// rounds and then a lower height in a second launch (4352 rows of a paired
+// launch of 80 column tiles, K = 3840: 16 tile rows in five rounds, then 256
+// rows as rf 4 in one). The model is good to a few percent, so what is not one
+// launch of 256-row tiles has to gain by it: a lower height 3% of one or two
+// rounds, 5% of more (16640 rows of [15360, 256], where both model alike: rf 6
+// 321 us, rf 8 259), a second launch 5% of a round (2560 rows of [10240, 3840]:
+// one launch 171.8 us, 240 tiles of rf 8 and then of rf 6 178.2). The paired
+// launch's lower heights gain a little more than modelled (400 rows: rf 6 76.6
+// us, rf 8 79.2) and its second launch starts inside the first one's end (a
+// feed-forward at 2048 rows 407 us with two, 416 with one): none, and 5% less.
+// With K in it 4096 rows of [10240, 64] take 28.5 us, by K = 3840's times 36.2.
+RowPlan plan_rows(int M, int tiles_n, int stages, bool pair) {
+  const int cus = device_cus();
+  const TileCost* const tiles = pair ? kPairTiles : kTiles;
+  const int nt = pair ? 3 : 4;
   const int tiles_m = (M + BM - 1) / BM;
-  auto rounds = [&](long long rows_of_tiles) {
-    return (double)((rows_of_tiles * tiles_n + cus - 1) / cus);
-  };
-  RowPlan best = {M, 8, 0.0};
-  double cost = rounds(tiles_m) * kTiles[0].us;
-  const int all = (int)rounds(tiles_m);
-  for (int k = 0; k < 4; ++k) {
-    // the tile rows that fill all - 1 - k rounds (k = 3: none)
-    const long long full = k < 3 ? (long long)(all - 1 - k) * cus / tiles_n : 0;
-    const int m1 = full < 0 ? 0 : full < tiles_m ? (int)full : tiles_m - 1;
-    const double head = m1 > 0 ? rounds(m1) * kTiles[0].us + 3.0 : 0.0;
-    for (const TileCost& t : kTiles) {
-      if (t.rf < rf_min) continue;
-      const double c = head + rounds((M - m1 * BM + 32 * t.rf - 1) / (32 * t.rf)) * t.us;
-      if (c < cost) {
-        cost = c;
-        best = {m1 * BM, t.rf, 0.0};
-      }
+  const long long all = ((long long)tiles_m * tiles_n + cus - 1) / cus;
+  // the rows past the first m1 tile rows at the lower height that takes least
+  auto rest = [&](int m1) {
+    RowPlan best = {m1 * BM, 8, -1.0};
+    for (int i = 1; i < nt; ++i) {
+      const int rows = M - m1 * BM, h = 32 * tiles[i].rf;
+      const double us = tiles_us(tiles[i], (long long)((rows + h - 1) / h) * tiles_n, stages);
+      if (best.us < 0.0 || us < best.us) best = {m1 * BM, tiles[i].rf, us};
     }
+    return best;
+  };
+  RowPlan best = {M, 8, tiles_us(tiles[0], (long long)tiles_m * tiles_n, stages)};
+  const RowPlan low = rest(0);
+  if (low.us < best.us * (all > 2 ? 0.95 : pair ? 1.0 : 0.97)) best = low;
+  RowPlan two = {0, 0, -1.0};
+  for (int k = 0; k < 3; ++k) {
+    // the tile rows that fill all - 1 - k rounds
+    const long long full = (all - 1 - k) * cus / tiles_n;
+    const int m1 = full < tiles_m ? (int)full : tiles_m - 1;
+    if (m1 <= 0) break;
+    RowPlan p = rest(m1);
+    p.us += tiles_us(tiles[0], (long long)m1 * tiles_n, stages);
+    if (two.us < 0.0 || p.us < two.us) two = p;
   }
-  best.us = cost;
+  const double round = tiles[0].full0 + tiles[0].full * stages;
+  if (two.us >= 0.0 && two.us < best.us + (pair ? 0.05 : -0.05) * round) best = two;
   return best;
+}
+
+// K stages of a launch, its longest LoRA tail's chunks counted as 5/8 of one.
+static int stages_of(const QprojArgs& a) {
+  int chunks = 0;
+  for (int i = 0; i < a.nseg; ++i) chunks = a.seg[i].chunks > chunks ? a.seg[i].chunks : chunks;
+  return a.K / BK + chunks * 5 / 8;
 }
 
 // The K split of a projection of few 256 x 256 tiles (the context refiner's
@@ -1253,9 +1287,13 @@ static RowPlan plan_rows(int M, int tiles_n, int rf_min) {
 // tiles would take (one round, at least 6 stages each), so the partials stay
 // within what they would take. [256, 3840] x [3840, 3840]: rf 2 in 4 slices, 24.6
 // us, where rf 8 in 10 took 30.7; 16 rows 14.1 against 18.6. 0: no split.
-static constexpr TileCost kStages[3] = {{8, 0.96}, {4, 0.57}, {2, 0.45}};
+struct StageCost {
+  int rf;
+  double us;
+};
+static constexpr StageCost kStages[3] = {{8, 0.96}, {4, 0.57}, {2, 0.45}};
 
-static double split_us(const TileCost& t, int M, int N, int K, int ks, int nw) {
+static double split_us(const StageCost& t, int M, int N, int K, int ks, int nw) {
   const int cus = device_cus();
   const int grid = ((M + 32 * t.rf - 1) / (32 * t.rf)) * ((N + BN - 1) / BN) * nw;
   return (double)((grid * ks + cus - 1) / cus) * ((K / BK + ks - 1) / ks) * t.us +
@@ -1272,7 +1310,7 @@ int qproj_split_plan(int M, int N, int K, int* rf) {
   if (kmax < 2) return 0;
   int best = 0;
   double cost = 0.0;
-  for (const TileCost& t : kStages)
+  for (const StageCost& t : kStages)
     for (int ks = 2; ks <= kmax; ++ks) {
       const double c = split_us(t, M, N, K, ks, 1);
       if (best == 0 || c < cost) {
@@ -1294,7 +1332,8 @@ bool qproj_merge_pays(int M, int N, int K, int nw) {
   int rf = 0;
   if (qproj_split_plan(M, N, K, &rf) > 0) return true;
   const int tiles_n = (N + BN - 1) / BN;
-  return plan_rows(M, nw * tiles_n, 2).us < 0.95 * nw * plan_rows(M, tiles_n, 2).us;
+  return plan_rows(M, nw * tiles_n, K / BK, false).us <
+         0.95 * nw * plan_rows(M, tiles_n, K / BK, false).us;
 }
 
 template <int BITS, bool SPLIT, int RF, int NW>
@@ -1400,12 +1439,13 @@ hipError_t launch_qproj_fast(int bits, const QprojArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(qproj_split_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
     return hipGetLastError();
   }
-  return launch_plan(a, plan_rows(a.M, (a.N + BN - 1) / BN, 2), [&](const QprojArgs& m, int rf) {
-    if (bits == 4)
-      launch_rows<4>(m, rf, s);
-    else
-      launch_rows<8>(m, rf, s);
-  });
+  return launch_plan(a, plan_rows(a.M, (a.N + BN - 1) / BN, stages_of(a), false),
+                     [&](const QprojArgs& m, int rf) {
+                       if (bits == 4)
+                         launch_rows<4>(m, rf, s);
+                       else
+                         launch_rows<8>(m, rf, s);
+                     });
 }
 
 hipError_t launch_qproj_merged(int bits, const QprojArgs& a, hipStream_t s) {
@@ -1418,7 +1458,7 @@ hipError_t launch_qproj_merged(int bits, const QprojArgs& a, hipStream_t s) {
       return hipErrorInvalidValue;
     QprojArgs m = a;
     double cost = 0.0;
-    for (const TileCost& t : kStages) {
+    for (const StageCost& t : kStages) {
       const double c = split_us(t, a.M, a.N, a.K, a.kslices, a.nw);
       if (cost == 0.0 || c < cost) {
         cost = c;
@@ -1437,7 +1477,7 @@ hipError_t launch_qproj_merged(int bits, const QprojArgs& a, hipStream_t s) {
                        0, s, a);
     return hipGetLastError();
   }
-  return launch_plan(a, plan_rows(a.M, a.nw * ((a.N + BN - 1) / BN), 2),
+  return launch_plan(a, plan_rows(a.M, a.nw * ((a.N + BN - 1) / BN), stages_of(a), false),
                      [&](const QprojArgs& m, int rf) {
                        if (bits == 4)
                          launch_merged_rows<4>(m, rf, s);
@@ -1452,7 +1492,7 @@ hipError_t launch_qproj_pair(int bits, const QprojArgs& a, hipStream_t s) {
       a.seg[0].chunks != a.seg_u.chunks || a.N % 8 != 0 || a.ldy % 8 != 0 ||
       (reinterpret_cast<uintptr_t>(a.y) & 15) != 0 || (bits != 4 && bits != 8))
     return hipErrorInvalidValue;
-  return launch_plan(a, plan_rows(a.M, (a.N + BN / 2 - 1) / (BN / 2), 4),
+  return launch_plan(a, plan_rows(a.M, (a.N + BN / 2 - 1) / (BN / 2), stages_of(a), true),
                      [&](const QprojArgs& m, int rf) {
                        if (bits == 4)
                          launch_pair_rows<4>(m, rf, s);
