@@ -1,0 +1,73 @@
+"""Projections under stream capture: what a captured call needs of the context's
+scratch, and what stays of it for the graph's replays when a later call grows
+it. Every replay is checked against the eager call, with eager work between."""
+import numpy as np
+import pytest
+import torch
+
+import ming_dit_amd as m
+from helpers import bf16, empty_bf16, from_dev, make_weight, randn, sync, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture()
+def cap():
+    """A context of its own (cold scratch) on a stream that can be captured."""
+    s = torch.cuda.Stream()
+    c = m.Ctx(0, s.cuda_stream)
+    c.stream = s
+    yield c
+    c.close()
+
+
+def _weight(ctx, seed, N, K, bits):
+    pack, _ = make_weight(seed, N, K, bits, std=1.0 / np.sqrt(K))
+    if bits == 16:
+        return m.QWeight.dense(ctx, pack["w"])
+    return m.QWeight.quantized(ctx, pack["codes"], pack["scales"], pack["biases"], bits)
+
+
+def _capture(ctx, fn):
+    sync()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=ctx.stream, capture_error_mode="thread_local"):
+        fn()
+    return g
+
+
+def test_growth_after_a_capture_keeps_the_graphs_scratch(cap):
+    """A split projection captured with a small partials' buffer still replays
+    to its own bits, into memory of its own, after a larger call grew it."""
+    M, N, K = 40, 512, 2048
+    q, big = _weight(cap, 4000, N, K, 4), _weight(cap, 4001, 3840, 3840, 4)
+    x = [to_dev(bf16(randn(4002 + i, (M, K)))) for i in range(3)]
+    xb, yb = to_dev(bf16(randn(4005, (256, 3840)))), empty_bf16(256, 3840)
+    xi, y = empty_bf16(M, K), empty_bf16(M, N)
+    sync()
+    want = []
+    for v in x:
+        cap.lin(q, v, y, M)
+        cap.synchronize()
+        want.append(from_dev(y))
+    cap.reset_engagement()
+    g = _capture(cap, lambda: cap.lin(q, xi, y, M))
+    assert cap.engagement()["gemm_split"] == 1
+    cap.lin(big, xb, yb, 256)                     # about 16 MB of partials
+    cap.synchronize()
+    first = from_dev(yb)
+    other = [torch.full((1 << 18,), 7, dtype=torch.int32, device="cuda") for _ in range(8)]
+    for v, w in zip(x, want):
+        xi.copy_(v)
+        y.zero_()
+        sync()
+        g.replay()
+        sync()
+        assert np.array_equal(from_dev(y), w)
+        cap.lin(big, xb, yb, 256)
+        cap.synchronize()
+        assert np.array_equal(from_dev(yb), first)
+    assert all(bool((o == 7).all()) for o in other)
+    del g
+    q.close()
+    big.close()

@@ -79,6 +79,10 @@ struct ming_ctx {
   size_t up_bytes = 0;
   void* part = nullptr;        // split-K partials of the stacked x.A GEMM
   size_t part_bytes = 0;
+  // a call under stream capture used `part`: the graph holds its address, so
+  // growing it keeps the old buffer (until the context goes) instead of freeing it
+  bool part_captured = false;
+  std::vector<void*> part_kept;
   int route = MING_ROUTE_AUTO;
   // device word raised by any fp16 copy that could not hold its value
   // (range_report); read and cleared at synchronization points
@@ -264,12 +268,25 @@ int ensure_scratch(ming_ctx* c, size_t bytes) {
   return MING_OK;
 }
 
+// Whether the context's stream is being captured (a query that fails, as on the
+// legacy stream beside another's capture, counts as yes).
+bool capturing(ming_ctx* c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 int ensure_part(ming_ctx* c, size_t bytes) {
   if (bytes <= c->part_bytes) return MING_OK;
   MING_HIP(hipStreamSynchronize(c->stream), "scratch grow sync");
-  if (c->part) (void)hipFree(c->part);
+  if (c->part && c->part_captured)
+    c->part_kept.push_back(c->part);
+  else if (c->part)
+    (void)hipFree(c->part);
   c->part = nullptr;
   c->part_bytes = 0;
+  c->part_captured = false;
   size_t want = std::max(bytes, (size_t)1 << 20);
   if (hipMalloc(&c->part, want) != hipSuccess)
     return fail(MING_ERR_ALLOC, "split-K partial scratch allocation failed");
@@ -501,6 +518,7 @@ int ming_ctx_destroy(ming_ctx* c) {
   if (c->vt) (void)hipFree(c->vt);
   if (c->up) (void)hipFree(c->up);
   if (c->part) (void)hipFree(c->part);
+  for (void* p : c->part_kept) (void)hipFree(p);
   if (c->range) (void)hipFree(c->range);
   for (auto& rec : c->recs) {
     (void)hipEventDestroy(rec.a);
@@ -1087,10 +1105,7 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
     // all projections' partials at once: a stream that is being captured, where
     // the buffer cannot grow, keeps to what it holds
     const size_t all = (size_t)n * split_ks[0] * M * qs[0]->N * 4;
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (all > c->part_bytes)
-      MING_HIP(hipStreamIsCapturing(c->stream, &st), "capture status");
-    merged = st == hipStreamCaptureStatusNone;
+    merged = all <= c->part_bytes || !capturing(c);
     if (merged) part_bytes = std::max(part_bytes, all);
   }
   // The fast route reads x as fp16 carrying the same (bf16) values: one
@@ -1124,7 +1139,10 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
     if (rc != MING_OK) return rc;
     if (t_bytes) T = (uint16_t*)c->scratch;
     if (xh_bytes) xh = (const uint16_t*)c->xh;
-    if (part_bytes) part = (float*)c->part;
+    if (part_bytes) {
+      part = (float*)c->part;
+      if (!c->part_captured) c->part_captured = capturing(c);
+    }
     if (up_bytes) up = (uint16_t*)c->up;
   }
 
