@@ -214,7 +214,9 @@ int ming_lin_bias(ming_ctx* ctx, const ming_qweight* qw, const uint16_t* x,
 /* ming_lin that allocates nothing. It has NO counterpart in the reference: it
  * is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). Same
- * arguments, kernels and bits as ming_lin; the call's scratch (the adapters'
+ * arguments, kernels and bits as ming_lin (which, for few rows of a dense
+ * weight, takes a kernel without partials where theirs cannot be allocated:
+ * captured before the context held them, or out of memory); the call's scratch (the adapters'
  * x.A intermediate, the fp16 copy of x, split-K partials) comes from one
  * static array of MING_NOALLOC_SCRATCH_BYTES per GPU, resident from the first
  * context on that GPU until the process ends. Refusals, before anything is

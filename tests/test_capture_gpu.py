@@ -1,6 +1,8 @@
 """Projections under stream capture: what a captured call needs of the context's
 scratch, and what stays of it for the graph's replays when a later call grows
 it. Every replay is checked against the eager call, with eager work between."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -71,3 +73,48 @@ def test_growth_after_a_capture_keeps_the_graphs_scratch(cap):
     del g
     q.close()
     big.close()
+
+
+def _cap_partials(ctx, nbytes):
+    f = m.lib()._ZN4ming15rt_set_part_capEP8ming_ctxm
+    f.argtypes, f.restype = [C.c_void_p, C.c_size_t], None
+    f(ctx.h, nbytes)
+
+
+@pytest.mark.parametrize("M,N,K,gated", [(203, 10240, 3840, False), (17, 4160, 1024, False),
+                                         (40, 1024, 2560, False), (130, 4160, 2048, True)])
+def test_dense_split_gives_way(orc, cap, M, N, K, gated):
+    """A dense projection of few rows that splits K runs unsplit, on the dense
+    route, where its partials have no room: under capture in a cold context,
+    and without memory for them."""
+    x, g = bf16(randn(4100 + M, (M, K))), bf16(randn(4101, (M, N)))
+    pack, w = make_weight(4102 + N, N, K, 16, std=1.0 / np.sqrt(K))
+    q = m.QWeight.dense(cap, pack["w"])
+    xd, gd, y = to_dev(x), to_dev(g), empty_bf16(M, N)
+    call = (lambda: cap.lin_swiglu(q, xd, gd, y, M)) if gated else (lambda: cap.lin(q, xd, y, M))
+    graph = _capture(cap, call)
+    seen = []
+    for _ in range(3):
+        y.zero_()
+        sync()
+        graph.replay()
+        sync()
+        seen.append(from_dev(y))
+    assert np.array_equal(seen[0], seen[1]) and np.array_equal(seen[0], seen[2])
+    _cap_partials(cap, 0)
+    call()
+    cap.synchronize()
+    assert np.array_equal(from_dev(y), seen[0])
+    _cap_partials(cap, 1 << 40)
+    call()
+    cap.synchronize()
+    ref = orc.proj(x, w)
+    if gated:
+        ref = orc.bf16_to_f32(orc.swiglu(g, orc.f32_to_bf16(ref)))
+    for got in (seen[0], from_dev(y)):
+        assert orc.rel_l2(orc.bf16_to_f32(got), ref) <= 2e-3
+    graph.replay()
+    sync()
+    assert np.array_equal(from_dev(y), seen[0])
+    del graph
+    q.close()

@@ -17,6 +17,8 @@ int rt_device(const ming_ctx* c);
 // models hold their context like weights do: it refuses to go first
 void rt_retain(ming_ctx* c);
 void rt_release(ming_ctx* c);
+// The partials' buffer stays at or below `bytes`, as if memory ended there (tests).
+void rt_set_part_cap(ming_ctx* c, size_t bytes);
 // the session log (ming_set_log_sink); level MING_LOG_WARN / MING_LOG_INFO
 void rt_log(int level, const std::string& msg);
 // a device copy of `bytes` host bytes on the context's device (NULL for 0)

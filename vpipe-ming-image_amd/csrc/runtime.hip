@@ -82,6 +82,7 @@ struct ming_ctx {
   // a call under stream capture used `part`: the graph holds its address, so
   // growing it keeps the old buffer (until the context goes) instead of freeing it
   bool part_captured = false;
+  size_t part_cap = SIZE_MAX;  // rt_set_part_cap
   std::vector<void*> part_kept;
   int route = MING_ROUTE_AUTO;
   // device word raised by any fp16 copy that could not hold its value
@@ -277,21 +278,46 @@ bool capturing(ming_ctx* c) {
   return true;
 }
 
-int ensure_part(ming_ctx* c, size_t bytes) {
-  if (bytes <= c->part_bytes) return MING_OK;
-  MING_HIP(hipStreamSynchronize(c->stream), "scratch grow sync");
+// The partials' buffer at `bytes`: false where it would have to grow and there
+// is no memory for it. `need`: what it holds now may go first (nothing of it is
+// in use once the stream is idle).
+bool grow_part(ming_ctx* c, size_t bytes, bool need) {
+  if (bytes <= c->part_bytes) return true;
+  const size_t want = std::max(bytes, (size_t)1 << 20);
+  auto take = [&]() -> void* {
+    void* p = nullptr;
+    if (want <= c->part_cap && hipMalloc(&p, want) == hipSuccess) return p;
+    (void)hipGetLastError();   // a launch's own check must not report it
+    return nullptr;
+  };
+  void* p = take();
+  if (!p && !need) return false;
+  if (hipStreamSynchronize(c->stream) != hipSuccess) {
+    if (p) (void)hipFree(p);
+    return false;
+  }
   if (c->part && c->part_captured)
     c->part_kept.push_back(c->part);
   else if (c->part)
     (void)hipFree(c->part);
-  c->part = nullptr;
-  c->part_bytes = 0;
+  c->part = p ? p : take();
+  c->part_bytes = c->part ? want : 0;
   c->part_captured = false;
-  size_t want = std::max(bytes, (size_t)1 << 20);
-  if (hipMalloc(&c->part, want) != hipSuccess)
-    return fail(MING_ERR_ALLOC, "split-K partial scratch allocation failed");
-  c->part_bytes = want;
-  return MING_OK;
+  return c->part != nullptr;
+}
+
+int ensure_part(ming_ctx* c, size_t bytes) {
+  if (bytes <= c->part_bytes) return MING_OK;
+  MING_HIP(hipStreamSynchronize(c->stream), "scratch grow sync");
+  if (grow_part(c, bytes, true)) return MING_OK;
+  return fail(MING_ERR_ALLOC, "split-K partial scratch allocation failed");
+}
+
+// Whether `bytes` of partials can be had, for a launch that has another form
+// without them: not where the buffer would have to grow under capture, or
+// cannot.
+bool part_room(ming_ctx* c, size_t bytes) {
+  return bytes <= c->part_bytes || (!capturing(c) && grow_part(c, bytes, false));
 }
 
 int ensure_xh(ming_ctx* c, size_t bytes) {
@@ -1064,12 +1090,19 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
                        (uint64_t)q->N * (uint64_t)K * 2 <= (1ull << 31);
     if (dense && live_segs[i] == 0 && tiles < 64 && q->N % 64 == 0 && o.ldy <= (1 << 30))
       dense_plan[i] = ming::dense_split_plan(M, q->N, K);
-    if (dense_plan[i].slices > 0) {
-      part_bytes = std::max(part_bytes, ming::lora_xa_part_bytes(M, q->N, dense_plan[i].slices,
-                                                                 dense_plan[i].tile));
-    } else if (dense && q->N % 8 == 0 && tail_fits[i]) {
-      dense_rf[i] = ming::dense_fast_rf(M, q->N);
+    if (dense_plan[i].slices > 1) {
+      // the dense route needs no partials: it takes the call where there is no
+      // room for them
+      const size_t want = std::max(
+          part_bytes,
+          ming::lora_xa_part_bytes(M, q->N, dense_plan[i].slices, dense_plan[i].tile));
+      if (carve || !tail_fits[i] || part_room(c, want))
+        part_bytes = want;
+      else
+        dense_plan[i].slices = 0;
     }
+    if (dense && dense_plan[i].slices == 0 && q->N % 8 == 0 && tail_fits[i])
+      dense_rf[i] = ming::dense_fast_rf(M, q->N);
     if (o.gate && !fast[i] && !dense_rf[i]) up_bytes = std::max(up_bytes, (size_t)M * q->N * 2);
   }
   // A SwiGLU's gate and up projections (the second gated by the first's
@@ -1823,6 +1856,7 @@ int rt_fail(int code, const std::string& why) { return fail(code, why); }
 int rt_ok() { return ok(); }
 int rt_device(const ming_ctx* c) { return c ? c->device : -1; }
 void rt_retain(ming_ctx* c) { c->live_weights += 1; }
+void rt_set_part_cap(ming_ctx* c, size_t bytes) { c->part_cap = bytes; }
 void rt_release(ming_ctx* c) { c->live_weights -= 1; }
 
 void rt_log(int level, const std::string& msg) {
