@@ -208,3 +208,10 @@ def plan_rows(M, tiles_n, stages, pair):
     f = m.lib()._ZN4ming9plan_rowsEiiib
     f.argtypes, f.restype = [C.c_int, C.c_int, C.c_int, C.c_bool], RowPlan
     return f(M, tiles_n, stages, pair)
+
+
+def split_plan(M, N, K):
+    """(slices, rows per tile) of a split projection; 0 slices: not split."""
+    rf = C.c_int()
+    ks = m.lib()._ZN4ming16qproj_split_planEiiiPi(M, N, K, C.byref(rf))
+    return ks, 32 * rf.value

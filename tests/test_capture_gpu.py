@@ -8,7 +8,9 @@ import pytest
 import torch
 
 import ming_dit_amd as m
-from helpers import bf16, empty_bf16, from_dev, make_weight, randn, sync, to_dev
+import test_block_gpu as tb
+from helpers import (bf16, build_block, empty_bf16, from_dev, make_weight, randn, split_plan, sync,
+                     to_dev)
 
 pytestmark = pytest.mark.gpu
 
@@ -118,3 +120,50 @@ def test_dense_split_gives_way(orc, cap, M, N, K, gated):
     assert np.array_equal(from_dev(y), seen[0])
     del graph
     q.close()
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_merged_split_gives_way(cap, monkeypatch, bits):
+    """A block's split q, k and v run as one launch where their partials fit
+    together, else (no memory, or captured before they did) as one each with the
+    same bits."""
+    rows, Hd = 700, 1024
+    monkeypatch.setattr(tb, "H", Hd)
+    monkeypatch.setattr(tb, "NH", Hd // 128)
+    _, gp, desc = build_block(cap, 4200, Hd, tb.F, tb.ADA, bits, False)
+    x = bf16(randn(4201, (rows, Hd)))
+    c, s = (to_dev(np.ascontiguousarray(t)) for t in tb.tables(rows))
+    src, xd = to_dev(x), to_dev(x)
+    ws = torch.empty(cap.block_workspace_bytes(tb.dims(), rows), dtype=torch.uint8, device="cuda")
+    call = lambda: cap.block_forward(desc, tb.dims(), xd, rows, c, s, None, tb.SCALES, ws)
+
+    def run(go):
+        xd.copy_(src)
+        sync()
+        go()
+        cap.synchronize()
+        sync()
+        return from_dev(xd)
+
+    def launches():
+        cap.set_profiling(True)
+        got = run(call)
+        n = cap.profile_collect()[f"qproj_fast.w{bits}"]["launches"]
+        cap.set_profiling(False)
+        return got, n
+
+    ks = split_plan(rows, Hd, Hd)[0]
+    assert ks >= 2
+    _cap_partials(cap, 2 * ks * rows * Hd * 4)      # two projections' partials
+    apart, n_apart = launches()
+    _cap_partials(cap, 1 << 40)
+    graph = _capture(cap, call)                     # the buffer still holds two
+    captured = [run(graph.replay) for _ in range(3)]
+    merged, n_merged = launches()
+    assert n_apart == n_merged + 2
+    for got in [merged, run(graph.replay)] + captured:
+        assert np.array_equal(got, apart)
+    del graph
+    for q in gp.values():
+        if hasattr(q, "close"):
+            q.close()

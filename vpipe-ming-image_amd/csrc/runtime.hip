@@ -1135,11 +1135,10 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
            (fast[0] ? ming::qproj_merge_pays(M, qs[0]->N, K, n)
                     : ming::dense_merge_pays(M, qs[0]->N, n));
   if (merged && split_ks[0] >= 2) {
-    // all projections' partials at once: a stream that is being captured, where
-    // the buffer cannot grow, keeps to what it holds
-    const size_t all = (size_t)n * split_ks[0] * M * qs[0]->N * 4;
-    merged = all <= c->part_bytes || !capturing(c);
-    if (merged) part_bytes = std::max(part_bytes, all);
+    // all projections' partials at once: one launch each where they have no room
+    const size_t all = std::max(part_bytes, (size_t)n * split_ks[0] * M * qs[0]->N * 4);
+    merged = part_room(c, all);
+    if (merged) part_bytes = all;
   }
   // The fast route reads x as fp16 carrying the same (bf16) values: one
   // conversion serves every projection here.
