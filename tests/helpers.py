@@ -215,3 +215,16 @@ def split_plan(M, N, K):
     rf = C.c_int()
     ks = m.lib()._ZN4ming16qproj_split_planEiiiPi(M, N, K, C.byref(rf))
     return ks, 32 * rf.value
+
+
+class DensePlan(C.Structure):
+    _fields_ = [("mr", C.c_int), ("cj", C.c_int), ("slices", C.c_int)]
+
+
+def dense_plan(M, N, K):
+    """(rows, columns, slices) of a dense projection's split plan; 0 slices: the
+    dense route."""
+    f = m.lib()._ZN4ming16dense_split_planEiii
+    f.restype = DensePlan
+    p = f(M, N, K)
+    return 64 * p.mr, 64 * p.cj, p.slices

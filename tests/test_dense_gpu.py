@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import ming_dit_amd as m
-from helpers import bf16, empty_bf16, from_dev, make_lora, make_weight, randn, sync, to_dev
+from helpers import bf16, dense_plan, empty_bf16, from_dev, make_lora, make_weight, randn, sync, to_dev
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-3
@@ -84,7 +84,7 @@ def test_dense_gated_few_tiles(ctx, M):
     qw.close()
 
 
-# Tiles of 64 x 64 to 256 x 128, one slice and several, more columns than the
+# Tiles of 128 x 64 and 128 x 128, one slice and several, more columns than the
 # adapters' group table holds.
 @pytest.mark.parametrize("M,N,K", [(9, 4160, 1024), (17, 256, 4096), (130, 1984, 640),
                                    (231, 1024, 2560), (300, 3840, 1024), (500, 704, 6400)])
@@ -103,3 +103,16 @@ def test_dense_few_tiles(ctx, orc, M, N, K):
     # slices are summed in order: the same bits again
     assert np.array_equal(plain, _run(ctx, "auto", lambda y: ctx.lin(qw, xd, y, M), M, N))
     qw.close()
+
+
+# Every tile of the plan, split and not (64 x 128 and 256 x 128 only split: unsplit
+# the plan finds others faster).
+@pytest.mark.parametrize("M,N,K,tile,split", [
+    (700, 1536, 192, (64, 64), False), (9, 4160, 10240, (64, 128), True),
+    (17, 1216, 640, (128, 64), False), (231, 832, 3840, (128, 64), True),
+    (1500, 2240, 1024, (128, 128), False), (9, 2112, 2560, (128, 128), True),
+    (130, 832, 10240, (256, 128), True), (4096, 256, 3840, (256, 128), True)])
+def test_dense_plan_tiles(ctx, orc, M, N, K, tile, split):
+    rows, cols, slices = dense_plan(M, N, K)
+    assert (rows, cols) == tile and (slices > 1 if split else slices == 1)
+    test_dense_few_tiles(ctx, orc, M, N, K)

@@ -3,7 +3,7 @@ CPU (without a device they count the MI355X's 256 CUs), through the library's
 own symbols."""
 import pytest
 
-from helpers import plan_rows
+from helpers import dense_plan, plan_rows
 
 SHAPES = [(M, tn, st) for M in (1, 63, 300, 700, 1280, 2085, 4352, 8320, 16640)
           for tn in (1, 8, 15, 40, 60, 80, 129) for st in (1, 4, 16, 60, 165)]
@@ -32,3 +32,13 @@ def test_row_plans_count_k():
     # a paired launch's 4352 rows: five whole rounds, then 128-row tiles
     p = plan_rows(4352, 80, 60, True)
     assert (p.rows_main, p.rf_rest) == (4096, 4)
+
+
+@pytest.mark.parametrize("M,N,K", [(203, 10240, 256), (1024, 3840, 64), (130, 15360, 128),
+                                   (1024, 2560, 256), (40, 10240, 64), (16, 64, 64)])
+def test_dense_plans_of_a_short_k(M, N, K):
+    """A tall tile's scattered stores are most of an unsplit launch of a few K
+    stages: 203 rows of [10240, 256] take 13.2 us on 256 x 128, 7.4 on the dense
+    route."""
+    rows, cols, slices = dense_plan(M, N, K)
+    assert slices == 0 or rows * cols <= 128 * 64

@@ -1549,19 +1549,25 @@ size_t lora_xa_part_bytes(int M, int n_cols, int kslices) {
 
 // A dense projection of fewer than 64 tiles of 256 x 256 through the x.A
 // kernel: its tile and slices by a time model, and whether that beats one
-// round of dense_fast.hip's 64-row tiles (about 5 us + 0.72 us a K stage). The
+// round of dense_fast.hip's 64-row tiles (about 4 us + 0.7 us a K stage). The
 // model, us: a start, the larger of the staged bytes at the tile's rate and
 // the stages of a block in its rounds, and for a split its reduce launch and
-// the f32 partials, written and read at 5 TB/s; within 10% of what it was
-// fitted to, 16-1024 rows at [2304..10240] x [2560..10240] with the weights
-// rotated through more than the 256 MB cache, as a forward meets them. 16 rows
-// of [3840, 3840]: 13.5 us (64 x 64 in 4 slices; 256 x 128 in 8: 19.2), 231 of
-// [3584, 2560]: 17.7 (128 x 64 in 2; 21.4), 1024 of [3840, 3840]: 42.2 (256 x
-// 128 in 2; 64-row tiles of dense_fast 48.5).
+// the f32 partials, written and read at 5 TB/s; unsplit, at least the tile's
+// own start (its scattered stores: the 256 x 128 one takes 10 us at one K
+// stage, the 64 x 64 one 4, dense_fast 4.5), stages and a part a round of
+// blocks. Measured with the weights rotated through more than the 256 MB
+// cache, as a forward meets them, over 9-1024 rows of [64..15360] x [64..10240]
+// in every tile and up to 12 slices; the plan against the best of those, us:
+// 16 rows of [3840, 3840] 15.3 (128 x 128 in 8; 64 x 64 in 4 13.4), 231 of
+// [3584, 2560] 17.7 (128 x 128 in 4, the best; 256 x 128 in 8 21.9), 1024 of
+// [3840, 3840] 42.0 (256 x 128 in 2, the best; dense_fast 48.3), 203 of [10240,
+// 256] 7.4 (dense_fast, the best; 256 x 128 unsplit 13.2). A gated call takes
+// the same plan, though its SwiGLU is then a launch of its own: its bits are
+// those of the plain call and ming_swiglu.
 DensePlan dense_split_plan(int M, int N, int K) {
   const int KT = K / 64;
   DensePlan best = {{4, 2}, 0};
-  double cost = 5.0 + 0.72 * KT;
+  double cost = 4.0 + 0.7 * KT;
   // the partials stay within what 256 x 128 tiles in one round would take
   const int tiles = ((M + 255) / 256) * ((N + 127) / 128);
   int kold = 256 / (tiles > 0 ? tiles : 1);
@@ -1573,11 +1579,12 @@ DensePlan dense_split_plan(int M, int N, int K) {
     XaTile t;
     int per_cu;                       // blocks a CU holds (LDS)
     double start_us, bytes_us, stage_us;
-  } cand[5] = {{{4, 2}, 1, 2.0, 14e6, 0.84},
-               {{2, 2}, 1, 3.0, 11.5e6, 0.65},
-               {{2, 1}, 2, 2.5, 10e6, 0.5},
-               {{1, 2}, 2, 5.0, 10e6, 0.5},
-               {{1, 1}, 3, 4.5, 10e6, 0.36}};
+    double direct0, direct;           // unsplit, a short K: start and stage
+  } cand[5] = {{{4, 2}, 1, 2.0, 14e6, 0.84, 8.8, 0.73},
+               {{2, 2}, 1, 3.0, 11.5e6, 0.65, 5.0, 0.52},
+               {{2, 1}, 2, 2.5, 10e6, 0.5, 3.9, 0.41},
+               {{1, 2}, 2, 5.0, 10e6, 0.5, 4.0, 0.43},
+               {{1, 1}, 3, 4.5, 10e6, 0.36, 3.1, 0.35}};
   for (const auto& c : cand) {
     const long long n = (long long)((M + 64 * c.t.mr - 1) / (64 * c.t.mr)) *
                         ((N + 64 * c.t.cj - 1) / (64 * c.t.cj));
@@ -1587,7 +1594,12 @@ DensePlan dense_split_plan(int M, int N, int K) {
       const double waits = (double)((n * ks + c.per_cu * cus - 1) / (c.per_cu * cus)) *
                            ((KT + ks - 1) / ks) * c.stage_us;
       double us = c.start_us + (staged > waits ? staged : waits);
-      if (ks > 1) us += 2.5 + 8.0 * ks * (double)M * N / 5e6;
+      if (ks > 1) {
+        us += 2.5 + 8.0 * ks * (double)M * N / 5e6;
+      } else {
+        const double own = c.direct0 + c.direct * KT + 1.2 * (double)n / cus;
+        us = us > own ? us : own;
+      }
       if (us < cost) {
         cost = us;
         best = {c.t, ks};
