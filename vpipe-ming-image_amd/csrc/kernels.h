@@ -297,6 +297,8 @@ hipError_t launch_qproj_fast(int bits, const QprojArgs& a, hipStream_t s);
 // all. qproj_merge_pays: whether that is less time than one launch each.
 hipError_t launch_qproj_merged(int bits, const QprojArgs& a, hipStream_t s);
 bool qproj_merge_pays(int M, int N, int K, int nw);
+// CUs of the current device, which the plans count rounds by (256 without one).
+int device_cus();
 // The rows of an unsplit launch: the first rows_main as 256-row tiles, the others
 // as tiles of 32 * rf_rest, and the time that takes by the plan's model. Each
 // output element is computed by the same MFMA sequence in every tile height, so

@@ -28,6 +28,8 @@
 //       k0..k3 one per byte and (w >> 4) & 0x0F0F0F0F holds k4..k7
 //   w8: codes[kt][n][fk][kk][2] two u32 = those 8 codes, bytes in k order
 //   sbf[kt][n] = fp16 scale | fp16 bias << 16
+#include <atomic>
+
 #include "common.h"
 #include "kernels.h"
 #include "lds_ring.h"
@@ -1179,19 +1181,18 @@ __global__ void bf16_to_f16_kernel(const uint16_t* x, long long ldx, uint16_t* y
 
 }  // namespace
 
-// CUs of the current device (the launch rounds are counted against it).
-static int device_cus() {
-  static int cached[64] = {};
+int device_cus() {
+  static std::atomic<int> cached[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         n <= 0)
       n = 256;
-    cached[dev] = n;
+    cached[dev].store(n, std::memory_order_relaxed);
   }
-  return cached[dev];
+  return n;
 }
 
 // Rows per tile. A launch of `tiles` tiles of 32*rf rows takes a start, a full
@@ -1305,7 +1306,7 @@ int qproj_split_plan(int M, int N, int K, int* rf) {
   const int tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   if (tiles <= 0 || tiles >= 64 || N % 4 != 0) return 0;
   const int KT = K / BK;
-  int kmax = 256 / tiles;
+  int kmax = device_cus() / tiles;
   if (kmax > KT / 6) kmax = KT / 6;
   if (kmax < 2) return 0;
   int best = 0;
@@ -1569,12 +1570,12 @@ DensePlan dense_split_plan(int M, int N, int K) {
   DensePlan best = {{4, 2}, 0};
   double cost = 4.0 + 0.7 * KT;
   // the partials stay within what 256 x 128 tiles in one round would take
+  const int cus = device_cus();
   const int tiles = ((M + 255) / 256) * ((N + 127) / 128);
-  int kold = 256 / (tiles > 0 ? tiles : 1);
+  int kold = cus / (tiles > 0 ? tiles : 1);
   const int kmax = KT / 8 > 1 ? KT / 8 : 1;
   if (kold > kmax) kold = kmax;
   const size_t room = lora_xa_part_bytes(M, N, kold, {4, 2});
-  const int cus = device_cus();
   const struct {
     XaTile t;
     int per_cu;                       // blocks a CU holds (LDS)
