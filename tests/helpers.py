@@ -228,3 +228,8 @@ def dense_plan(M, N, K):
     f.restype = DensePlan
     p = f(M, N, K)
     return 64 * p.mr, 64 * p.cj, p.slices
+
+
+def merged_split_rows(M, N, K, slices, nw=3):
+    """Rows per tile of nw split projections as one launch."""
+    return 32 * m.lib()._ZN4ming21qproj_merged_split_rfEiiiii(M, N, K, slices, nw)

@@ -116,3 +116,33 @@ def test_dense_plan_tiles(ctx, orc, M, N, K, tile, split):
     rows, cols, slices = dense_plan(M, N, K)
     assert (rows, cols) == tile and (slices > 1 if split else slices == 1)
     test_dense_few_tiles(ctx, orc, M, N, K)
+
+
+@pytest.mark.parametrize("M,K", [(70, 256), (2100, 640)])
+def test_dense_segments(ctx, M, K):
+    """A concatenated dense weight, its segments with adapters of their own and
+    none, gives each part's own bits (64- and 192-row tiles)."""
+    print(f"case dense segments M={M} K={K}", flush=True)
+    parts, Ns, ranks = [], (256, 512, 1032), ((16, 64), (), (40,))
+    for i, N in enumerate(Ns):
+        q = m.QWeight.dense(ctx, make_weight(10400 + i, N, K, 16, std=1.0 / np.sqrt(K))[0]["w"])
+        for s, r in enumerate(ranks[i]):
+            q.bind_lora(s, *make_lora(10410 + 2 * (4 * i + s), N, K, r))
+        parts.append(q)
+    fused = m.QWeight.concat(ctx, parts)
+    assert fused.n_segments == 3
+    xd, sc = to_dev(bf16(randn(10450, (M, K)))), [0.7, -0.4] + [0.0] * 6
+    got = _run(ctx, "auto", lambda y: ctx.lin(fused, xd, y, M, sc), M, sum(Ns))
+    general = _run(ctx, "general", lambda y: ctx.lin(fused, xd, y, M, sc), M, sum(Ns))
+    n0 = 0
+    for i, N in enumerate(Ns):
+        want = _run(ctx, "auto", lambda y: ctx.lin(parts[i], xd, y, M, sc), M, N)
+        mine = got[:, n0:n0 + N]
+        if ranks[i]:
+            assert np.array_equal(mine, want)
+        else:
+            # alone, with no adapter, the part may split K
+            assert np.array_equal(mine, general[:, n0:n0 + N])
+        n0 += N
+    for q in parts + [fused]:
+        q.close()

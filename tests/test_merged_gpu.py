@@ -6,15 +6,15 @@ import numpy as np
 import pytest
 
 import test_block_gpu as tb
-from helpers import bf16, build_block, from_dev, randn
+from helpers import (bf16, build_block, from_dev, make_lora, merged_split_rows, randn,
+                     split_plan)
 
 pytestmark = pytest.mark.gpu
 BUCKET = {4: "qproj_fast.w4", 8: "qproj_fast.w8", 16: "qproj.dense"}
 
 
-# H = 512 (no K split): six column tiles in the merged launch. 1000 rows take
-# 64-row tiles, 3000 128, 5600 192, 8300 256, 11000 two 256-row rounds and 64
-# (dense: 192). H = 1024 splits K in two.
+# H = 512 (no K split): six column tiles in the merged launch, the heights of 1000
+# to 11000 rows. H = 1024 splits K in two, in 64- and 128-row tiles.
 @pytest.mark.parametrize("bits,Hd,rows", [
     (4, 512, 1000), (4, 512, 3000), (4, 512, 5600), (4, 512, 8300), (4, 512, 11000),
     (8, 512, 1000), (8, 512, 8300), (8, 512, 11000),
@@ -25,6 +25,11 @@ def test_merged_qkv_bits(ctx, monkeypatch, bits, Hd, rows):
     monkeypatch.setattr(tb, "H", Hd)
     monkeypatch.setattr(tb, "NH", Hd // 128)
     _, gp, desc = build_block(ctx, 970, Hd, tb.F, tb.ADA, bits, False)
+    _equals_its_calls(ctx, gp, desc, bits, Hd, rows)
+
+
+def _equals_its_calls(ctx, gp, desc, bits, Hd, rows):
+    """The block with its q, k and v merged against its public calls."""
     x = bf16(randn(971, (rows, Hd)))
     c, s = tb.tables(rows)
     ctx.set_profiling(True)
@@ -45,3 +50,29 @@ def test_merged_qkv_bits(ctx, monkeypatch, bits, Hd, rows):
     for q in gp.values():
         if hasattr(q, "close"):
             q.close()
+
+
+# The merged split in 256-row tiles, as the caption block's 203 rows take it.
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("Hd,rows", [(1024, 1360), (3840, 203)])
+def test_merged_split_high_tiles(ctx, monkeypatch, bits, Hd, rows):
+    slices = split_plan(rows, Hd, Hd)[0]
+    assert slices >= 2 and merged_split_rows(rows, Hd, Hd, slices) == 256
+    test_merged_qkv_bits(ctx, monkeypatch, bits, Hd, rows)
+
+
+# q, k and v with different adapters: a tail of its own each (k a longer one, v
+# none, dense one of 32 ranks), which also moves each one's K slices.
+@pytest.mark.parametrize("bits,Hd,rows", [(4, 512, 1000), (8, 512, 3000), (16, 512, 1000),
+                                          (4, 1024, 203), (8, 1024, 700)])
+def test_merged_different_adapters(ctx, monkeypatch, bits, Hd, rows):
+    print(f"case merged adapters bits={bits} H={Hd} rows={rows}", flush=True)
+    monkeypatch.setattr(tb, "H", Hd)
+    monkeypatch.setattr(tb, "NH", Hd // 128)
+    _, gp, desc = build_block(ctx, 975, Hd, tb.F, tb.ADA, bits, False)
+    assert tb.SCALES[0] and tb.SCALES[3]
+    gp["k"].bind_lora(0, *make_lora(976, Hd, Hd, 100))
+    # a dense v without any might split K by itself, apart from the others
+    for slot in (0, 3) if bits != 16 else (3,):
+        gp["v"].unbind_lora(slot)
+    _equals_its_calls(ctx, gp, desc, bits, Hd, rows)

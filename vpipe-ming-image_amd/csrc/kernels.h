@@ -311,6 +311,8 @@ struct RowPlan {
 RowPlan plan_rows(int M, int tiles_n, int stages, bool pair);
 // K slices of a projection of few tiles, and its tile height (0: no split).
 int qproj_split_plan(int M, int N, int K, int* rf);
+// The tile height (rf) of nw projections' merged launch of those slices.
+int qproj_merged_split_rf(int M, int N, int K, int kslices, int nw);
 // The gate and up projections of a SwiGLU in one launch (the fields after
 // `range` in QprojArgs): each 256 x 256 tile holds 128 columns of each, so
 // the gate's output meets the up projection's in LDS and only

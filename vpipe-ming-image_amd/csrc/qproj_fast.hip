@@ -1323,6 +1323,19 @@ int qproj_split_plan(int M, int N, int K, int* rf) {
   return best;
 }
 
+int qproj_merged_split_rf(int M, int N, int K, int kslices, int nw) {
+  int rf = 8;
+  double cost = 0.0;
+  for (const StageCost& t : kStages) {
+    const double c = split_us(t, M, N, K, kslices, nw);
+    if (cost == 0.0 || c < cost) {
+      cost = c;
+      rf = t.rf;
+    }
+  }
+  return rf;
+}
+
 // One launch each against one for all. Split: the merged one fills its rounds
 // of blocks, and is two launches where there were two each (a w4 block at 203
 // rows 312 us with three, 288 with one). Unsplit: where the rounds of all are
@@ -1458,14 +1471,7 @@ hipError_t launch_qproj_merged(int bits, const QprojArgs& a, hipStream_t s) {
         a.K / BK < a.kslices)
       return hipErrorInvalidValue;
     QprojArgs m = a;
-    double cost = 0.0;
-    for (const StageCost& t : kStages) {
-      const double c = split_us(t, a.M, a.N, a.K, a.kslices, a.nw);
-      if (cost == 0.0 || c < cost) {
-        cost = c;
-        m.split_rf = t.rf;
-      }
-    }
+    m.split_rf = qproj_merged_split_rf(a.M, a.N, a.K, a.kslices, a.nw);
     if (bits == 4)
       launch_merged_split<4>(m, s);
     else
