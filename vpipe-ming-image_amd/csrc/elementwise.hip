@@ -255,8 +255,8 @@ __device__ __forceinline__ float row_min(float v) {
 // codes, scales and biases, so group gi needs no row or column. HBM-bound: 16
 // lanes take a group, 4 consecutive weights each, so a wave reads 1 KB and
 // writes 128 B (w4) or 256 B (w8) contiguous, four groups in flight a lane
-// (one thread a group, striding 256 B from its neighbour, took 607 us for
-// [10240, 3840] at w4; this takes 40.6, 4.4 TB/s). V16: w is 16-byte aligned.
+// (one thread a group, striding 256 B from its neighbour, took 596 us for
+// [10240, 3840] at w4; this takes 40, 4.5 TB/s). V16: w is 16-byte aligned.
 template <int BITS, bool V16>
 __global__ __launch_bounds__(256) void quantize_kernel(const float* w, long long groups,
                                                        uint32_t* codes, uint16_t* scales,

@@ -194,7 +194,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
       (MULTI && wsel > 0 ? a.more[wsel - 1].sb : upw ? a.sb_u : a.sb) + (long long)kt0 * a.N;
 
   // DMA sources for this lane, per stage (advance by k).
-  // x tile: wave issues chunks q = 8*wave + i; lane p = 64q + lane.
+  // x tile: wave issues chunks q = XD*wave + i; lane p = 64q + lane.
   // Byte offsets from the stage's base (the host keeps every operand
   // within 2 GiB of its base, so they fit 31 bits whether the hardware reads
   // the offset as signed or unsigned).
@@ -226,7 +226,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   sn = sn < nlast ? sn : nlast;
   const uint32_t soff = (uint32_t)sn * 4u;
 
-  // The stage's DMAs in three groups (x rows 0-127, x rows 128-255, codes +
+  // The stage's DMAs in three groups (the wave's x DMAs in two halves, codes +
   // (s, b)), issued one group per k16 step of the stage before.
   auto issue_grp = [&](int g, int kt, const uint4* B) {
     if (g < 2) {
@@ -252,7 +252,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[j][i][r] = 0.0f;
 
-  // Stage state in registers: the code words and (s, b) of the wave's two
+  // Stage state in registers: the code words and (s, b) of the wave's
   // n-tiles, and the current k16 step's operands.
   uint4 wc[JT][CPR / 2];
   half2v s2[JT], b2[JT];
@@ -285,7 +285,7 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
 
   // One stage, software-pipelined across the stage boundary. Steps 0-2
   // read and dequantize the next step's fragments beside the current
-  // step's 16 MFMAs and issue one DMA group of stage kt+2 into Pv (the
+  // step's MFMAs and issue one DMA group of stage kt+2 into Pv (the
   // buffer stage kt-1 left). Between steps 2 and 3 the wave waits for its
   // stage kt+1 DMAs and the workgroup meets at the barrier: stage kt+1 is
   // in LDS and nobody reads stage kt's buffer again. Step 3's MFMAs then
@@ -431,40 +431,24 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
     uint32_t toff[TD];
     uint32_t boff[BD];
     int bc[BD];
-    if constexpr (TD == BD) {
 #pragma unroll
-      for (int i = 0; i < BD; ++i) {
-        const int p = 64 * (BD * wave + i) + lane;
-        const int row = p >> 2;
-        const int c = (p & 3) ^ ((row >> 2) & 3);
-        int m = m0 + row;
-        m = m < mlast ? m : mlast;
-        toff[i] = (uint32_t)(((long long)m * a.ldt + t_col0 + 8 * c) * 2);
-        int n = n0 + (PAIR ? (row & 127) : row);
-        n = n < seg_ne - 1 ? n : seg_ne - 1;
-        boff[i] = (uint32_t)((long long)(n - seg_nb) * ldb * 2);
-        bc[i] = c;
-      }
-    } else {
+    for (int i = 0; i < TD; ++i) {
+      const int p = 64 * (TD * wave + i) + lane;
+      const int row = p >> 2;
+      const int c = (p & 3) ^ ((row >> 2) & 3);
+      int m = m0 + row;
+      m = m < mlast ? m : mlast;
+      toff[i] = (uint32_t)(((long long)m * a.ldt + t_col0 + 8 * c) * 2);
+    }
 #pragma unroll
-      for (int i = 0; i < TD; ++i) {
-        const int p = 64 * (TD * wave + i) + lane;
-        const int row = p >> 2;
-        const int c = (p & 3) ^ ((row >> 2) & 3);
-        int m = m0 + row;
-        m = m < mlast ? m : mlast;
-        toff[i] = (uint32_t)(((long long)m * a.ldt + t_col0 + 8 * c) * 2);
-      }
-#pragma unroll
-      for (int i = 0; i < BD; ++i) {
-        const int p = 64 * (BD * wave + i) + lane;
-        const int row = p >> 2;
-        const int c = (p & 3) ^ ((row >> 2) & 3);
-        int n = n0 + (PAIR ? (row & 127) : row);
-        n = n < seg_ne - 1 ? n : seg_ne - 1;
-        boff[i] = (uint32_t)((long long)(n - seg_nb) * ldb * 2);
-        bc[i] = c;
-      }
+    for (int i = 0; i < BD; ++i) {
+      const int p = 64 * (BD * wave + i) + lane;
+      const int row = p >> 2;
+      const int c = (p & 3) ^ ((row >> 2) & 3);
+      int n = n0 + (PAIR ? (row & 127) : row);
+      n = n < seg_ne - 1 ? n : seg_ne - 1;
+      boff[i] = (uint32_t)((long long)(n - seg_nb) * ldb * 2);
+      bc[i] = c;
     }
     // A lane's 16 bytes are the 8 ranks of one group; the chunk's four groups
     // are wave-uniform (scalar loads).
@@ -580,12 +564,12 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
   }
 
   if constexpr (PAIR) {
-    // The gate's and the up projection's bf16 outputs meet in LDS, 128 rows
-    // at a time: wave w writes its 64 columns to region w (as below), and
-    // after the barrier wave w reads column half c = w & 1 of rows
-    // [64 (w >> 1), +64) from the gate's region c and the up projection's
-    // region 2 + c, and writes y = bf16(silu(g) * u) and its fp16 copy: the
-    // bits of the gate's own epilogue followed by the gated one.
+    // The gate's and the up projection's bf16 outputs meet in LDS, up to 128
+    // rows at a time: regions 0 and 1 hold the gate's two column halves, 2 and 3
+    // the up projection's (a wave a region, or two with eight waves), and after
+    // the barrier wave w reads half w & 1 of both over its share of the rows and
+    // writes y = bf16(silu(g) * u) and its fp16 copy: the bits of the gate's own
+    // epilogue followed by the gated one.
     const int rg = wave * JT / 2;   // the 64-column region this wave writes
     uint2* const Ew = reinterpret_cast<uint2*>(region(rg));
     const uint4* const Eg = region(wave & 1);
@@ -643,12 +627,12 @@ __device__ __forceinline__ void qproj_fast_body(const QprojArgs& a) {
     return;
   }
 
-  // Epilogue through LDS: each wave converts its 64 columns x 128 rows at a
-  // time to bf16 in its own 16 KB region (rows of 128 B, chunks swizzled by
-  // (row >> 1) & 7 so both the 8-B writes and the 16-B reads are
-  // conflict-free), then stores whole 128-B row segments, 8 rows per
-  // instruction. Only the wave itself touches its region, and LDS accesses
-  // of one wave complete in order, so no barrier is needed inside.
+  // Epilogue through LDS: a 16 KB region holds 64 columns x up to 128 rows in
+  // bf16 (rows of 128 B, chunks swizzled by (row >> 1) & 7 so both the 8-B
+  // writes and the 16-B reads are conflict-free), stored as whole 128-B row
+  // segments, 8 rows per instruction. With four waves only the wave itself
+  // touches its region, and LDS accesses of one wave complete in order, so no
+  // barrier is needed inside; with eight, two waves share one.
   const int rg = wave * JT / 2;   // the 64-column region this wave writes and stores from
   uint4* const E = region(rg);
   const bool st16 = (a.ldy & 7) == 0 && (reinterpret_cast<uintptr_t>(yout) & 15) == 0;
@@ -785,20 +769,20 @@ __global__ void qproj_split_reduce_kernel(const QprojArgs a) {
 }
 
 // ---- T = x . A_live^T * coef: the adapters' stacked down-projection --------
-// Block tile 256 rows x 128 stacked ranks. Four MFMA waves in 2 x 2, each
-// 128 rows x 64 ranks (4 x 2 tiles of v_mfma_f32_32x32x16_bf16, D[rank][row],
-// so a lane owns one row and 4 consecutive ranks per register quad), and a
-// DMA-only wave beside each on its SIMD: a global_load_lds holds the wave
-// that issues it for ~16 cycles its MFMAs do not hide, so no MFMA wave
-// issues one. Split-K over kslices so the grid is about one round of the
-// chip; slice s writes f32 partials P[s] and lora_xa_reduce_kernel sums the
-// slices in a fixed order (no atomics: the bits do not depend on timing).
-// With one slice the block writes T directly. A three-stage ring of [x 32 KB
-// | A 16 KB] filled by inline-asm DMA, one barrier a stage, which every wave
-// passes once: before it the DMA waves issue stage t + 2 into the buffer
-// stage t - 1 left and wait until stage t + 1 has landed; the MFMA waves
-// have then finished every read of stage t (steps 0-2 read it; step 3,
-// after the barrier, reads stage t + 1's first fragments).
+// Block tile 64*MR rows x 64*CJ stacked ranks. Four MFMA waves in 2 x 2, each
+// 32*MR rows x 32*CJ ranks (MR x CJ tiles of v_mfma_f32_32x32x16_bf16,
+// D[rank][row], so a lane owns one row and 4 consecutive ranks per register
+// quad), and a DMA-only wave beside each on its SIMD: a global_load_lds holds
+// the wave that issues it for ~16 cycles its MFMAs do not hide, so no MFMA wave
+// issues one. Split-K over kslices so the grid is about one round of the chip;
+// slice s writes f32 partials P[s] and lora_xa_reduce_kernel sums the slices in
+// a fixed order (no atomics: the bits do not depend on timing). With one slice
+// the block writes T directly. A three-stage ring of [x | A] (48 KB a stage at
+// 256 x 128) filled by inline-asm DMA, one barrier a stage, which every wave
+// passes once: before it the DMA waves issue stage t + 2 into the buffer stage
+// t - 1 left and wait until stage t + 1 has landed; the MFMA waves have then
+// finished every read of stage t (steps 0-2 read it; step 3, after the barrier,
+// reads stage t + 1's first fragments).
 template <int MR, int CJ>
 __global__ __launch_bounds__(512, 1) void lora_xa_fast_kernel(const LoraXaArgs a, float* part,
                                                               int kslices) {
