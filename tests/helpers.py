@@ -233,3 +233,15 @@ def dense_plan(M, N, K):
 def merged_split_rows(M, N, K, slices, nw=3):
     """Rows per tile of nw split projections as one launch."""
     return 32 * m.lib()._ZN4ming21qproj_merged_split_rfEiiiii(M, N, K, slices, nw)
+
+
+class XaTile(C.Structure):
+    _fields_ = [("mr", C.c_int), ("cj", C.c_int)]
+
+
+def xa_tile(M, n_cols, K, slices):
+    """(rows, columns) of the adapters' x.A tile."""
+    f = m.lib()._ZN4ming7xa_tileEiiii
+    f.restype = XaTile
+    t = f(M, n_cols, K, slices)
+    return 64 * t.mr, 64 * t.cj

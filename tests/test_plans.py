@@ -3,7 +3,7 @@ CPU (without a device they count the MI355X's 256 CUs), through the library's
 own symbols."""
 import pytest
 
-from helpers import dense_plan, plan_rows
+from helpers import dense_plan, plan_rows, xa_tile
 
 SHAPES = [(M, tn, st) for M in (1, 63, 300, 700, 1280, 2085, 4352, 8320, 16640)
           for tn in (1, 8, 15, 40, 60, 80, 129) for st in (1, 4, 16, 60, 165)]
@@ -42,3 +42,13 @@ def test_dense_plans_of_a_short_k(M, N, K):
     route."""
     rows, cols, slices = dense_plan(M, N, K)
     assert slices == 0 or rows * cols <= 128 * 64
+
+
+def test_xa_tiles_at_half_a_chip():
+    """The adapters' x.A: 256 x 128 tiles from half a chip of them on (512 ranks at
+    8320 rows: 65 us, 64-row tiles 74), a block more where K is short."""
+    assert xa_tile(8320, 512, 3840, 1) == (256, 128)
+    assert xa_tile(16640, 256, 10240, 1) == (256, 128)
+    assert xa_tile(16640, 256, 3840, 1) == (64, 128)
+    assert xa_tile(16384, 256, 10240, 1) == (64, 128)
+    assert xa_tile(4352, 64, 3840, 3) == (64, 64)

@@ -329,8 +329,9 @@ hipError_t launch_repack_fast(int bits, const uint32_t* codes,
 int lora_xa_fast_slices(int M, int n_cols, int K);
 // Bytes of f32 partials launch_lora_xa_fast needs for kslices > 1 (whole
 // tiles per slice, in the kernel's accumulator order); 0 otherwise.
-size_t lora_xa_part_bytes(int M, int n_cols, int kslices);
+size_t lora_xa_part_bytes(int M, int n_cols, int K, int kslices);
 size_t lora_xa_part_bytes(int M, int n_cols, int kslices, XaTile t);
+XaTile xa_tile(int M, int n_cols, int K, int kslices);
 // The same kernel as a plain split-K bf16 GEMM y = x . W^T of a dense W
 // [N][K] of few tiles: its tile and slices, 0 slices where dense_fast.hip's
 // kernel is the faster one.

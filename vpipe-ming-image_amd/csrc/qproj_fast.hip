@@ -1519,12 +1519,15 @@ int lora_xa_fast_slices(int M, int n_cols, int K) {
 // 256 x 128 one stages the fewest bytes and is taken where its blocks fill
 // half the chip; a narrow stack or a short x leaves it on a few CUs (one
 // adapter of rank 16 at 4352 rows: 51 blocks, 42.3 us with its reduce) where
-// 64-row tiles spread out (19.9). Measured at 16-512 ranks, 100-16640 rows:
-// 512 ranks at 1493 rows (168 blocks) 23.5 against 25.5, at 1024 (112) 24.1
-// against 21.8.
-static XaTile xa_tile(int M, int n_cols, int kslices) {
+// 64-row tiles spread out (19.9). Measured over 64-1536 ranks, 300-16640 rows
+// and K = 256 to 10240: up to 128 of its blocks the 64-row tiles take 0.4 to
+// 0.9 of its time, from 132 it takes 0.75 to 1 of theirs (512 ranks at 8320
+// rows, 132 blocks, K = 3840: 65.4 us against 73.8; at K = 256 1.1); at 130
+// (256 ranks, 16640 rows) theirs are 8% faster at K = 3840, 2-6% slower at
+// 10240, where a block stages more before it stores.
+XaTile xa_tile(int M, int n_cols, int K, int kslices) {
   const long long blocks = (long long)((M + 255) / 256) * ((n_cols + 127) / 128) * kslices;
-  if (blocks >= 136) return {4, 2};
+  if (blocks > (K > 4096 ? 128 : 130)) return {4, 2};
   return n_cols <= 64 ? XaTile{1, 1} : XaTile{1, 2};
 }
 
@@ -1534,8 +1537,8 @@ size_t lora_xa_part_bytes(int M, int n_cols, int kslices, XaTile t) {
   return (size_t)kslices * (((size_t)M + xr - 1) / xr) * (((size_t)n_cols + xc - 1) / xc) *
          (xr * xc * 4);
 }
-size_t lora_xa_part_bytes(int M, int n_cols, int kslices) {
-  return lora_xa_part_bytes(M, n_cols, kslices, xa_tile(M, n_cols, kslices));
+size_t lora_xa_part_bytes(int M, int n_cols, int K, int kslices) {
+  return lora_xa_part_bytes(M, n_cols, kslices, xa_tile(M, n_cols, K, kslices));
 }
 
 // A dense projection of fewer than 64 tiles of 256 x 256 through the x.A
@@ -1621,7 +1624,7 @@ static hipError_t launch_xa_tiles(const LoraXaArgs& a, float* part, int kslices,
 hipError_t launch_lora_xa_fast(const LoraXaArgs& a, float* part, int kslices,
                                hipStream_t s) {
   if (a.M <= 0 || a.n_cols <= 0) return hipSuccess;
-  const XaTile t = a.ident ? a.tile : xa_tile(a.M, a.n_cols, kslices);
+  const XaTile t = a.ident ? a.tile : xa_tile(a.M, a.n_cols, a.K, kslices);
   switch (10 * t.mr + t.cj) {
     case 11: return launch_xa_tiles<1, 1>(a, part, kslices, s);
     case 12: return launch_xa_tiles<1, 2>(a, part, kslices, s);

@@ -1061,7 +1061,7 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
   const bool xa_fast = t_cols > 0 && c->route != MING_ROUTE_GENERAL && ldx % 8 == 0 &&
                        (uint64_t)M * (uint64_t)ldx * 2 <= (1ull << 31) && xa_fits;
   const int xa_ks = xa_fast ? ming::lora_xa_fast_slices(M, t_cols, K) : 1;
-  size_t part_bytes = ming::lora_xa_part_bytes(M, t_cols, xa_ks);
+  size_t part_bytes = ming::lora_xa_part_bytes(M, t_cols, K, xa_ks);
   // Which projections take the fast route. It addresses each operand as a
   // 64-bit base plus 32-bit byte offsets: x (fp16 copy, row stride K), T and
   // every B stack must fit.
