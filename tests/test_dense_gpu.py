@@ -84,6 +84,22 @@ def test_dense_gated_few_tiles(ctx, M):
     qw.close()
 
 
+# The output in x's own memory: no wider than x, and wider at a stride past both.
+@pytest.mark.parametrize("M,N,K,ld", [(600, 1032, 1088, 1088), (2100, 2056, 2112, 2112),
+                                      (300, 1032, 576, 1664)])
+def test_dense_gated_over_x(ctx, M, N, K, ld):
+    pack, _ = make_weight(9410, N, K, 16, std=1.0 / np.sqrt(K))
+    qw = m.QWeight.dense(ctx, pack["w"])
+    xd, g = to_dev(bf16(randn(9411, (M, ld)))), to_dev(bf16(randn(9412, (M, N))))
+    want = empty_bf16(M, N)
+    sync()
+    ctx.lin_swiglu(qw, xd, g, want, M, ldx=ld)
+    ctx.lin_swiglu(qw, xd, g, xd, M, ldx=ld, ldo=ld)
+    sync()
+    assert np.array_equal(from_dev(xd)[:, :N], from_dev(want))
+    qw.close()
+
+
 # Tiles of 128 x 64 and 128 x 128, one slice and several, more columns than the
 # adapters' group table holds.
 @pytest.mark.parametrize("M,N,K", [(9, 4160, 1024), (17, 256, 4096), (130, 1984, 640),

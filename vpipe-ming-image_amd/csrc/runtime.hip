@@ -886,6 +886,14 @@ struct LinOut {
   const uint16_t* bias = nullptr;   // dense weights only (ming_lin_bias)
 };
 
+// Two bf16 matrices of M rows whose address ranges share a byte.
+static bool overlap(const uint16_t* a, int64_t lda, int na, const uint16_t* b, int64_t ldb,
+                    int nb, int M) {
+  const uint64_t a0 = (uint64_t)(uintptr_t)a, b0 = (uint64_t)(uintptr_t)b;
+  return a0 < b0 + 2 * (uint64_t)((M - 1) * ldb + nb) &&
+         b0 < a0 + 2 * (uint64_t)((M - 1) * lda + na);
+}
+
 // n projections over the same x [M][K] (q, k, v; w1, w3): x is converted to
 // fp16 once for all of them (`xh_src`, when set, is that copy already made,
 // row stride K), and every live adapter of every one of them goes into ONE
@@ -1114,7 +1122,10 @@ static int lin_multi(ming_ctx* c, int n, const ming_qweight* const* qs, const Li
       else
         dense_plan[i].slices = 0;
     }
-    if (dense && dense_plan[i].slices == 0 && q->N % 8 == 0 && tail_fits[i])
+    // fused, a gated output lands while other tiles still read x: one that
+    // shares memory with x goes by the plane
+    if (dense && dense_plan[i].slices == 0 && q->N % 8 == 0 && tail_fits[i] &&
+        !(o.gate && overlap(o.y, o.ldy, q->N, x, ldx, K, M)))
       dense_rf[i] = ming::dense_fast_rf(M, q->N);
     if (o.gate && !fast[i] && !dense_rf[i]) up_bytes = std::max(up_bytes, (size_t)M * q->N * 2);
   }
